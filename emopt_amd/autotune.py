@@ -8,7 +8,9 @@ itself (``emf_time_steps``), on its own grid, materials and CPML, and the
 fastest is kept.  Every candidate computes bit-for-bit the same fields (the
 parity tests check each one), so tuning never changes results.  Winners are
 cached per (grid, complex eps, uniform mu) in memory and, when a path is given,
-in a JSON file.
+in a JSON file.  Where solves run resident (emf_resident; 3 to 5 times faster
+than any step kernel) a winner of another kind than the two passes is reported
+but not applied, which leaves them so.
 
 Batches: steps per graph replay, z planes per work-group and persistent
 work-groups per CU are timed on a sample of the batch's members (a fixed
@@ -48,6 +50,15 @@ def _load(path):
     return {}
 
 
+def _apply(L, h, best):
+    """Select the step kernel `best`, unless that ends resident solves."""
+    boxes = ctypes.c_int()
+    L.emf_set_tuning(h, *SOLVE_CANDIDATES[0])
+    L.emf_resident(h, ctypes.byref(boxes))
+    if boxes.value == 0 or best[0] == 1:
+        L.emf_set_tuning(h, *best)
+
+
 def tune_solver(sim, candidates=None, steps=40, warmup=8, cache_path=None, verbose=False):
     """Time each candidate on `sim` and apply the fastest; returns
     (best candidate, {candidate: ms per step}).  The solver's fields and CPML
@@ -56,7 +67,9 @@ def tune_solver(sim, candidates=None, steps=40, warmup=8, cache_path=None, verbo
     disk = _load(cache_path)
     if key in _cache or key in disk:
         best = tuple(_cache.get(key) or disk[key])
-        sim._lib.emf_set_tuning(sim._h, *best)
+        if not sim._mats_ready:
+            sim.build()
+        _apply(sim._lib, sim._h, best)
         return best, {}
     if not sim._mats_ready:
         sim.build()
@@ -77,7 +90,7 @@ def tune_solver(sim, candidates=None, steps=40, warmup=8, cache_path=None, verbo
         if verbose:
             print("tune %s: %.4f ms/step" % (cand, times[cand]))
     best = min(times, key=times.get)
-    L.emf_set_tuning(h, *best)
+    _apply(L, h, best)
     L.emf_reset_pml(h)
     L.emf_zero_fields(h)
     _cache[key] = list(best)

@@ -10,6 +10,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <climits>
 #include <cmath>
@@ -18,6 +19,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <condition_variable>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -25,6 +27,7 @@
 
 #include "../../include/emfdtd.h"
 #include "batch.hpp"
+#include "resident.hpp"
 #include "material.hpp"
 
 using namespace emf;
@@ -212,6 +215,13 @@ struct emf_solver {
 
     double2 *scratch = nullptr;
     size_t scratch_n = 0;
+
+    // resident steps (resident.hpp): off once a launch stalled, or by emf_set_resident
+    bool res_off = false;
+    int res_spin = RES_SPIN;
+    unsigned long long *res_halo = nullptr;
+    size_t res_halo_n = 0;
+    bool res_halo_clean = false;   // every slot EMPTY
 
     // weight planes of emf_interp_dot: per id, six optional complex planes
     static constexpr int kWeightSets = 8;
@@ -995,6 +1005,184 @@ int phasor3(emf_solver *s, int slot, double t0, double t1, double t2)
     return EMF_OK;
 }
 
+// ---- resident steps (resident.hpp) ---------------------------------------
+
+// How a grid is split into boxes: GX x GY x GZ of them, NZ planes per thread.
+struct ResPlan {
+    int NZ = 0, GX = 0, GY = 0, GZ = 0, BX = 0, BY = 0, threads = 0;
+    size_t lds = 0;
+    int boxes() const { return GX * GY * GZ; }
+};
+
+constexpr size_t kResLds = 160 * 1024;
+
+int res_max_planes(const emf_solver *s) { return s->ceps || !s->mu_uniform ? 3 : 5; }
+
+// Fills the plan for boxes of this split; false where the kernel cannot take it.
+bool res_split(const emf_solver *s, int GX, int GY, int GZ, ResPlan &r)
+{
+    r.GX = GX; r.GY = GY; r.GZ = GZ;
+    r.BX = (s->Nx + GX - 1) / GX; r.BY = (s->Ny + GY - 1) / GY; r.NZ = (s->Nz + GZ - 1) / GZ;
+    if (r.NZ > res_max_planes(s) || r.BX > RES_W || r.BY > RES_W || r.BX * r.BY > RES_T ||
+        (r.BX + 1) * (r.BY + 1) > RES_PL)
+        return false;
+    // a thread per column, and RES_ITEMS halo slots of the x and y faces per thread
+    const int items = 2 * r.NZ * (r.BX + r.BY);
+    r.threads = (std::max(r.BX * r.BY, (items + RES_ITEMS - 1) / RES_ITEMS) + 63) / 64 * 64;
+    r.lds = res_lds(r.NZ, r.BX, r.BY);
+    return r.threads <= RES_T && r.lds <= kResLds;
+}
+
+// The split with the least estimated time per step, if the grid fits one.  The
+// estimate follows measured splits of twelve grids from 24x20x16 to 120x80x60
+// (us per step, as chosen / best of 14 splits tried: 64x64x64 5.1 / 4.9,
+// 120x80x60 7.8 / 7.8, 100x70x64 7.2 / 7.2, 48x44x100 4.8 / 4.6): work is the
+// cells of a box in whole waves, and an x face costs more than its share, one
+// 8-byte store a line where the other faces fill theirs.  Every grid that fits
+// runs resident: the two passes took 12.8 us on 24x20x16 (resident 2.5), 18.5 on
+// 64x64x64 and 25.8 on 120x80x60.
+bool resident_plan(const emf_solver *s, int ncu, ResPlan &best)
+{
+    if (s->res_off || s->kind != 1 || s->wide || s->Nx < 2 || s->Ny < 2 || s->Nz < 2) return false;
+    double bt = 1e30;
+    for (int GZ = 1; GZ <= std::min(ncu, s->Nz); ++GZ) {
+        if ((s->Nz + GZ - 1) / GZ > res_max_planes(s)) continue;
+        for (int GY = 1; GY <= std::min(ncu / GZ, s->Ny); ++GY)
+            for (int GX = 1; GX <= std::min(ncu / (GZ * GY), s->Nx); ++GX) {
+                ResPlan r;
+                if (!res_split(s, GX, GY, GZ, r)) continue;
+                const double t = 0.15 * r.NZ * (r.threads / 64) + 0.02 * r.NZ * r.BY;
+                if (t < bt) { bt = t; best = r; }
+            }
+    }
+    return bt < 1e30;
+}
+
+// Work-groups of resident launches in flight on a device: all of them have to
+// be able to run at once, so no more than the CUs are admitted together.
+struct ResGate {
+    std::mutex m;
+    std::condition_variable cv;
+    int used = 0, ncu = 0;
+};
+ResGate g_res_gate[64];
+
+struct ResHold {
+    ResGate *g = nullptr;
+    int n = 0;
+    void take(ResGate &gate, int boxes)
+    {
+        std::unique_lock<std::mutex> lk(gate.m);
+        gate.cv.wait(lk, [&] { return gate.used + boxes <= gate.ncu; });
+        gate.used += boxes;
+        g = &gate;
+        n = boxes;
+    }
+    void give()
+    {
+        if (!g) return;
+        { std::lock_guard<std::mutex> lk(g->m); g->used -= n; }
+        g->cv.notify_all();
+        g = nullptr;
+    }
+    ~ResHold() { give(); }
+};
+
+int res_cus(int dev, int *ncu)
+{
+    *ncu = 0;
+    if (dev < 0 || dev >= 64) return EMF_OK;
+    ResGate &gate = g_res_gate[dev];
+    std::lock_guard<std::mutex> lk(gate.m);
+    if (!gate.ncu)
+        HIPCHK(hipDeviceGetAttribute(&gate.ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    *ncu = gate.ncu;
+    return EMF_OK;
+}
+
+int res_ready(emf_solver *s, const ResPlan &r)
+{
+    const size_t n = (size_t)4 * r.boxes() * res_slots(r.NZ);
+    if (n > s->res_halo_n) {
+        dfree(s->res_halo);
+        s->res_halo_n = 0;
+        CHECK(dalloc(&s->res_halo, n));
+        s->res_halo_n = n;
+        s->res_halo_clean = false;
+    }
+    if (!s->res_halo_clean) {
+        hipLaunchKernelGGL(k_fill_slots, dim3(grid1d((long long)s->res_halo_n, 256)), dim3(256), 0,
+                           s->stream, s->res_halo, (long long)s->res_halo_n);
+        HIPCHK(hipGetLastError());
+        s->res_halo_clean = true;
+    }
+    return EMF_OK;
+}
+
+template <int NZ, bool CE, bool MU>
+int res_launch_t(emf_solver *s, const ResPlan &r, const ResArgs &R, const FusedArgs &A,
+                 const Geo &g, const int *done)
+{
+    auto K = k_resident<NZ, CE, MU>;
+    static std::atomic<bool> lds_set{ false };
+    if (!lds_set.exchange(true))
+        HIPCHK(hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)kResLds));
+    hipLaunchKernelGGL(K, dim3(r.boxes()), dim3(r.threads), r.lds, s->stream, R, A, g, done);
+    HIPCHK(hipGetLastError());
+    return EMF_OK;
+}
+
+template <bool CE, bool MU>
+int res_launch_nz(emf_solver *s, const ResPlan &r, const ResArgs &R, const FusedArgs &A,
+                  const Geo &g, const int *done)
+{
+    switch (r.NZ) {
+    case 1: return res_launch_t<1, CE, MU>(s, r, R, A, g, done);
+    case 2: return res_launch_t<2, CE, MU>(s, r, R, A, g, done);
+    case 3: return res_launch_t<3, CE, MU>(s, r, R, A, g, done);
+    }
+    if constexpr (!CE && !MU) {
+        if (r.NZ == 4) return res_launch_t<4, CE, MU>(s, r, R, A, g, done);
+        return res_launch_t<5, CE, MU>(s, r, R, A, g, done);
+    }
+    EMF_FAIL(EMF_ERR_ARG, "no resident kernel for %d planes", r.NZ);
+}
+
+// Steps n .. n + count - 1 with the state resident, RES_STEPS per launch.
+int res_steps(emf_solver *s, const ResPlan &r, long long n, long long count, const int *done)
+{
+    PassTab th, te;
+    CHECK(refresh_tables(s, &th, &te));
+    CHECK(refresh_sources(s));
+    CHECK(res_ready(s, r));
+    ResArgs R;
+    R.GX = r.GX; R.GY = r.GY; R.GZ = r.GZ; R.BX = r.BX; R.BY = r.BY;
+    R.spin = s->res_spin;
+    R.halo = s->res_halo;
+    R.conv = s->conv;
+    R.blk = s->src_desc;
+    R.nsrc = (int)s->srcs.size();
+    src_union(s, R.ub);
+    const FusedArgs A = make_args(s, 0, 0);
+    const Geo g = s->geo();
+    while (count > 0) {
+        R.nsteps = (int)std::min<long long>(count, RES_STEPS);
+        for (int q = 0; q < R.nsteps; ++q) {
+            const double t = (double)(n + q) * s->dt, tE = ((double)(n + q) + 0.5) * s->dt;
+            const double f[6] = { sin(t), cos(t), env_at(s, t), sin(tE), cos(tE), env_at(s, tE) };
+            memcpy(R.fac[q], f, sizeof(f));
+        }
+        if (s->ceps && !s->mu_uniform) CHECK((res_launch_nz<true, true>(s, r, R, A, g, done)));
+        else if (s->ceps) CHECK((res_launch_nz<true, false>(s, r, R, A, g, done)));
+        else if (!s->mu_uniform) CHECK((res_launch_nz<false, true>(s, r, R, A, g, done)));
+        else CHECK((res_launch_nz<false, false>(s, r, R, A, g, done)));
+        n += R.nsteps;
+        count -= R.nsteps;
+    }
+    return EMF_OK;
+}
+
 // Convergence sample points: arange(0, I*J*K, int(I*J*K/nconv)) over the
 // padded array (emopt/fdtd.py:411-413).  On one rank a ghost-face sample reads
 // the opposite face's outermost layer (the periodic self-exchange of
@@ -1024,6 +1212,120 @@ int build_samples(emf_solver *s)
                           hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));   // cells is a temporary
     s->nsamples = (int)cells.size();
+    return EMF_OK;
+}
+
+// What a run of the solve loop ended with.
+struct SolveRun {
+    long long n0 = 0;
+    int status = 0;
+    int stalled = 0;               // a resident launch gave up: the results are void
+    int nchecks = 0;
+    double a_change = 0, phi_change = 0;
+};
+
+// The solve loop from zero fields: steps until convergence (or fixed_n0 steps),
+// the two snapshots and the phasors.  plan: resident steps, null: the passes.
+int solve_run(emf_solver *s, int slot, double rtol, double nmax, long long Tn, long long fixed_n0,
+              const ResPlan *plan, SolveRun &run)
+{
+    run = SolveRun();
+    // reset CPML and fields (emopt/fdtd.py:1016-1018); set 0 holds step 0
+    set_current(s, 0);
+    CHECK(reset_psi(s));
+    HIPCHK(hipMemsetAsync(s->Ev[0], 0, 3 * s->n * sizeof(double), s->stream));
+    HIPCHK(hipMemsetAsync(s->Hv[0], 0, 3 * s->n * sizeof(double), s->stream));
+    HIPCHK(hipMemsetAsync(s->conv, 0, sizeof(ConvState), s->stream));
+    const double amp_rtol = rtol, phi_rtol = sqrt(rtol);
+    int *dflag = &s->conv->done;
+    // steps [from, from + count); the state after n steps lives in set
+    // from_set(n) (fused) or set 0
+    auto steps = [&](long long from, long long count, const int *done) -> int {
+        if (plan) return res_steps(s, *plan, from, count, done);
+        for (long long q = from; q < from + count; ++q) CHECK(step(s, q, done, from_set(s, q, 0, 0)));
+        return EMF_OK;
+    };
+
+    long long n = 0;
+    if (fixed_n0 >= 0) {
+        CHECK(steps(0, fixed_n0, nullptr));
+        n = fixed_n0;
+        run.status = 2;
+    } else {
+        // The loop breaks at the first step index n > nmax (emopt/fdtd.py:1054).
+        long long n_stop = nmax < 0 ? 0 : (long long)floor(nmax) + 1;
+        const int LOOK = 2;               // chunks in flight before the first flag is read
+        std::vector<std::pair<long long, hipEvent_t>> pend;
+        int ring = 0;
+        while (true) {
+            while ((int)pend.size() < LOOK && Tn > 0 && n + Tn <= n_stop) {
+                // steps after convergence are gated off by dflag and leave the state as is
+                CHECK(steps(n, Tn, dflag));
+                long long nchk = n + Tn - 1;
+                int slotf = ring++ % 32;
+                const int ps = from_set(s, n + Tn, 0, 0);   // set holding E after step nchk
+                hipLaunchKernelGGL(k_conv_check, dim3(1), dim3(64), 0, s->stream, s->Eb[ps][0],
+                                   s->Eb[ps][1], s->Eb[ps][2], s->samples, s->nsamples,
+                                   (double)nchk * s->dt, amp_rtol, phi_rtol, nchk, s->conv,
+                                   s->hist, s->hist_cap, (int *)nullptr);
+                HIPCHK(hipGetLastError());
+                // done and stalled
+                HIPCHK(hipMemcpyAsync(&s->done_host[2 * slotf], dflag, 2 * sizeof(int),
+                                      hipMemcpyDeviceToHost, s->stream));
+                hipEvent_t ev;
+                HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+                HIPCHK(hipEventRecord(ev, s->stream));
+                pend.push_back({ n, ev });
+                n += Tn;
+            }
+            if (pend.empty()) {
+                // fewer than Tn steps remain before nmax: run them and stop
+                CHECK(steps(n, n_stop - n, dflag));
+                n = std::max(n, n_stop);
+                run.status = 1;
+                break;
+            }
+            auto front = pend.front();
+            pend.erase(pend.begin());
+            HIPCHK(hipEventSynchronize(front.second));
+            (void)hipEventDestroy(front.second);
+            int slotf = (ring - 1 - (int)pend.size()) % 32;
+            if (s->done_host[2 * slotf + 1]) { run.stalled = 1; break; }
+            if (s->done_host[2 * slotf]) {
+                n = front.first + Tn;
+                break;
+            }
+        }
+        for (auto &pe : pend) {
+            (void)hipEventSynchronize(pe.second);
+            (void)hipEventDestroy(pe.second);
+        }
+        if (run.stalled) return EMF_OK;
+    }
+    // capture / two more Tn-step runs / phasor (emopt/fdtd.py:1156-1194)
+    long long n0 = n;
+    set_current(s, from_set(s, n0, 0, 0));
+    CHECK(capture(s, slot, 0));
+    CHECK(steps(n0, Tn, nullptr));
+    set_current(s, from_set(s, n0 + Tn, 0, 0));
+    CHECK(capture(s, slot, 1));
+    CHECK(steps(n0 + Tn, Tn, nullptr));
+    set_current(s, from_set(s, n0 + 2 * Tn, 0, 0));
+    CHECK(phasor3(s, slot, (double)n0 * s->dt, (double)(n0 + Tn) * s->dt,
+                  (double)(n0 + 2 * Tn) * s->dt));
+    // the scalars at the end of the state
+    struct { double a_change, phi_change; int done, stalled, nchecks; } cs;
+    static_assert(offsetof(ConvState, done) == offsetof(ConvState, a_change) + 16 &&
+                  offsetof(ConvState, nchecks) == offsetof(ConvState, done) + 8, "tail layout");
+    HIPCHK(hipMemcpyAsync(&cs, &s->conv->a_change, offsetof(ConvState, nchecks) + sizeof(int) -
+                                                       offsetof(ConvState, a_change),
+                          hipMemcpyDeviceToHost, s->stream));
+    HIPCHK(hipStreamSynchronize(s->stream));
+    run.n0 = n0;
+    run.stalled = cs.stalled;
+    run.nchecks = cs.nchecks;
+    run.a_change = cs.a_change;
+    run.phi_change = cs.phi_change;
     return EMF_OK;
 }
 
@@ -1158,6 +1460,7 @@ int emf_delete(emf_solver *s)
         dfree(s->samples);
         dfree(s->hist);
         dfree(s->scratch);
+        dfree(s->res_halo);
         for (int w = 0; w < emf_solver::kWeightSets; ++w)
             for (int q = 0; q < 6; ++q) dfree(s->wplane[w][q]);
         if (s->done_host) (void)hipHostFree(s->done_host);
@@ -1601,99 +1904,41 @@ int emf_solve(emf_solver *s, int slot, double rtol, double nmax, int64_t Tn, int
         s->hist_cap = (int)cap;
     }
     auto t_start = std::chrono::steady_clock::now();
-    // reset CPML and fields (emopt/fdtd.py:1016-1018); set 0 holds step 0
-    set_current(s, 0);
-    CHECK(reset_psi(s));
-    for (int c = 0; c < 3; ++c) {
-        HIPCHK(hipMemsetAsync(s->E[c], 0, s->n * sizeof(double), s->stream));
-        HIPCHK(hipMemsetAsync(s->H[c], 0, s->n * sizeof(double), s->stream));
-    }
-    HIPCHK(hipMemsetAsync(s->conv, 0, sizeof(ConvState), s->stream));
-    const double amp_rtol = rtol, phi_rtol = sqrt(rtol);
-    int *dflag = &s->conv->done;
-    // the state after n steps lives in set from_set(n) (fused) or set 0
-
-    long long n = 0;
-    int status = 0;
-    if (fixed_n0 >= 0) {
-        for (long long q = 0; q < fixed_n0; ++q) CHECK(step(s, q, nullptr, from_set(s, q, 0, 0)));
-        n = fixed_n0;
-        status = 2;
+    ResPlan plan;
+    int ncu = 0;
+    CHECK(res_cus(s->dev, &ncu));
+    SolveRun run;
+    if (resident_plan(s, ncu, plan)) {
+        ResHold hold;
+        hold.take(g_res_gate[s->dev], plan.boxes());
+        const int rc = solve_run(s, slot, rtol, nmax, Tn, fixed_n0, &plan, run);
+        if (rc != EMF_OK || run.stalled) (void)hipStreamSynchronize(s->stream);
+        hold.give();
+        CHECK(rc);
+        if (run.stalled) {
+            // the work-groups of a launch did not run together: from the start with the passes
+            s->res_off = true;
+            s->res_halo_clean = false;
+            CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
+        }
     } else {
-        // The loop breaks at the first step index n > nmax (emopt/fdtd.py:1054).
-        long long n_stop = nmax < 0 ? 0 : (long long)floor(nmax) + 1;
-        const int LOOK = 2;               // chunks in flight before the first flag is read
-        std::vector<std::pair<long long, hipEvent_t>> pend;
-        int ring = 0;
-        while (true) {
-            while ((int)pend.size() < LOOK && Tn > 0 && n + Tn <= n_stop) {
-                // steps after convergence are gated off by dflag and leave the state as is
-                for (long long q = 0; q < Tn; ++q) CHECK(step(s, n + q, dflag, from_set(s, n + q, 0, 0)));
-                long long nchk = n + Tn - 1;
-                int slotf = ring++ % 64;
-                const int ps = from_set(s, n + Tn, 0, 0);   // set holding E after step nchk
-                hipLaunchKernelGGL(k_conv_check, dim3(1), dim3(64), 0, s->stream, s->Eb[ps][0],
-                                   s->Eb[ps][1], s->Eb[ps][2], s->samples, s->nsamples,
-                                   (double)nchk * s->dt, amp_rtol, phi_rtol, nchk, s->conv,
-                                   s->hist, s->hist_cap, (int *)nullptr);
-                HIPCHK(hipGetLastError());
-                HIPCHK(hipMemcpyAsync(&s->done_host[slotf], dflag, sizeof(int),
-                                      hipMemcpyDeviceToHost, s->stream));
-                hipEvent_t ev;
-                HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-                HIPCHK(hipEventRecord(ev, s->stream));
-                pend.push_back({ n, ev });
-                n += Tn;
-            }
-            if (pend.empty()) {
-                // fewer than Tn steps remain before nmax: run them and stop
-                for (; n < n_stop; ++n) CHECK(step(s, n, dflag, from_set(s, n, 0, 0)));
-                status = 1;
-                break;
-            }
-            auto front = pend.front();
-            pend.erase(pend.begin());
-            HIPCHK(hipEventSynchronize(front.second));
-            (void)hipEventDestroy(front.second);
-            int slotf = (ring - 1 - (int)pend.size()) % 64;
-            if (s->done_host[slotf]) {
-                n = front.first + Tn;
-                break;
-            }
-        }
-        for (auto &pe : pend) {
-            (void)hipEventSynchronize(pe.second);
-            (void)hipEventDestroy(pe.second);
-        }
+        CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
     }
-    // capture / two more Tn-step runs / phasor (emopt/fdtd.py:1156-1194)
-    long long n0 = n;
-    set_current(s, from_set(s, n0, 0, 0));
-    CHECK(capture(s, slot, 0));
-    for (long long q = n0; q < n0 + Tn; ++q) CHECK(step(s, q, nullptr, from_set(s, q, 0, 0)));
-    set_current(s, from_set(s, n0 + Tn, 0, 0));
-    CHECK(capture(s, slot, 1));
-    for (long long q = n0 + Tn; q < n0 + 2 * Tn; ++q) CHECK(step(s, q, nullptr, from_set(s, q, 0, 0)));
-    set_current(s, from_set(s, n0 + 2 * Tn, 0, 0));
-    CHECK(phasor3(s, slot, (double)n0 * s->dt, (double)(n0 + Tn) * s->dt,
-                  (double)(n0 + 2 * Tn) * s->dt));
-    ConvState cs;
-    HIPCHK(hipMemcpyAsync(&cs, s->conv, sizeof(ConvState), hipMemcpyDeviceToHost, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
     auto t_end = std::chrono::steady_clock::now();
-    s->nhist = std::min(cs.nchecks, s->hist_cap);
+    s->nhist = std::min(run.nchecks, s->hist_cap);
     // the loop runs on past non-finite samples (emopt/fdtd.py:1050-1052,
     // 1137-1138) and stops at Nmax: say so when the last check saw them
-    if (status == 1 && cs.nchecks > 0 && !(std::isfinite(cs.a_change) && std::isfinite(cs.phi_change)))
-        status = 3;
+    if (run.status == 1 && run.nchecks > 0 &&
+        !(std::isfinite(run.a_change) && std::isfinite(run.phi_change)))
+        run.status = 3;
     if (info) {
-        info->n0 = n0;
+        info->n0 = run.n0;
         info->Tn = Tn;
-        info->steps = n0 + 2 * Tn;
-        info->status = status;
-        info->nchecks = cs.nchecks;
-        info->a_change = cs.a_change;
-        info->phi_change = cs.phi_change;
+        info->steps = run.n0 + 2 * Tn;
+        info->status = run.status;
+        info->nchecks = run.nchecks;
+        info->a_change = run.a_change;
+        info->phi_change = run.phi_change;
         info->seconds = std::chrono::duration<double>(t_end - t_start).count();
     }
     return EMF_OK;
@@ -2445,6 +2690,27 @@ int emf_set_tuning(emf_solver *s, int kind, int tyg, int zc, int order)
     s->tyg = tyg;
     s->zc = zc;
     s->order = order;
+    return EMF_OK;
+}
+
+int emf_set_resident(emf_solver *s, int on, int spin)
+{
+    LOCK(s);
+    if ((on != 0 && on != 1) || spin < 0) EMF_FAIL(EMF_ERR_ARG, "on must be 0 or 1, spin >= 0");
+    s->res_off = !on;
+    s->res_spin = spin > 0 ? spin : RES_SPIN;
+    return EMF_OK;
+}
+
+int emf_resident(emf_solver *s, int *boxes)
+{
+    LOCK(s);
+    if (!boxes) EMF_FAIL(EMF_ERR_ARG, "null output");
+    CHECK(check_ready(s));
+    ResPlan plan;
+    int ncu = 0;
+    CHECK(res_cus(s->dev, &ncu));
+    *boxes = resident_plan(s, ncu, plan) ? plan.boxes() : 0;
     return EMF_OK;
 }
 

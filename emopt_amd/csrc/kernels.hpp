@@ -265,6 +265,7 @@ struct ConvState {
     double t0, t1, t2;
     double a_change, phi_change;
     int done;
+    int stalled;                  // a resident launch gave up waiting for a neighbour
     int nchecks;
 };
 

@@ -374,6 +374,19 @@ EMF_API int emf_set_tuning(emf_solver *s, int kind, int tyg, int zc, int order);
  * batch members take only smaller grids.  No counterpart in the reference. */
 EMF_API int emf_set_wide_offsets(emf_solver *s, int force);
 
+/* Resident steps: a solve (emf_solve) with step kernel kind 1 whose grid fits
+ * the chip's registers (up to about 655,000 cells with real eps and uniform
+ * mu, 393,000 otherwise) takes many steps per launch with its state on chip.
+ * on = 0 keeps such a solve on the step kernels; spin > 0 bounds the polls for
+ * a neighbour's data before the launch counts as stalled and the solve is
+ * repeated with the step kernels (0: the default, some seconds).  The fields
+ * agree to roundoff either way.  No counterpart in the reference. */
+EMF_API int emf_set_resident(emf_solver *s, int on, int spin);
+
+/* *boxes = work-groups of the resident launches this solver's next emf_solve
+ * would use, 0 where it uses the step kernels. */
+EMF_API int emf_resident(emf_solver *s, int *boxes);
+
 /* Work-group shape of the H pass of the two-pass kernels (kinds 1 and 3):
  * rows (waves) per work-group tyg in {1, 2, 4, 8} and z planes per work-group
  * zc >= 1; 0 keeps the E pass's value (emf_set_tuning).  A launch shape only:
