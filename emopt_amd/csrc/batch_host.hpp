@@ -9,7 +9,10 @@
 // them between replays -- the graphs are never re-captured and record no
 // memset or copy nodes.
 //
-// Lanes: the members are split into cache-sized groups, and `lanes` groups
+// A member whose grid fits on chip (resident.hpp) is not stepped by these
+// kernels: a run until members finish gives it its own resident solve.
+//
+// Lanes: the other members are split into cache-sized groups, and `lanes` groups
 // are stepped at once, each by its own stream, copy of the table and graph.
 // Lanes never step the same group, so they share no data; the kernels of one
 // lane fill the CUs that another lane's launch leaves idle at its tail, and
@@ -22,6 +25,9 @@ struct BatchSlot {
     emf_solver *s = nullptr;
     int slot = 0;
     bool finished = false;
+    bool tiled = false;                 // stepped by the batch's kernels (else resident, on its own)
+    double rtol = 0, nmax = 0;          // as admitted
+    long long Tn = 0, fixed_n0 = -1;
     double *fac = nullptr;              // device per-step factors
     emf_solve_info info{};
     std::chrono::steady_clock::time_point t_add;
@@ -31,6 +37,7 @@ struct BatchSlot {
 }  // namespace
 
 constexpr int BATCH_LANES_MAX = 4;
+constexpr int BATCH_OWN = 4;             // resident solves at once
 
 struct emf_batch {
     std::mutex mtx;
@@ -80,7 +87,7 @@ int batch_upload_table(emf_batch *b)
     // arrival order): the first group then holds the oldest solves
     int order[BATCH_MAX], na = 0;
     for (int m = 0; m < BATCH_MAX; ++m)
-        if (b->sl[m].s && !b->sl[m].finished) order[na++] = m;
+        if (b->sl[m].s && b->sl[m].tiled && !b->sl[m].finished) order[na++] = m;
     std::sort(order, order + na, [&](int x, int y) { return b->sl[x].seq < b->sl[y].seq; });
     for (int q = 0; q < na; ++q) {
         const int m = order[q];
@@ -193,6 +200,118 @@ void batch_finish(emf_batch *b, int m, const BState &st)
         std::chrono::duration<double>(std::chrono::steady_clock::now() - q.t_add).count();
     std::lock_guard<std::mutex> lks(q.s->mtx);
     q.s->nhist = std::min(st.nchecks, q.s->hist_cap);
+}
+
+// Make slot `id` a member stepped by the batch's kernels: its state reset, its
+// step factors, descriptor and device state uploaded (the caller rewrites the
+// table).  The caller holds the solver's lock.
+int batch_tile(emf_batch *b, int id)
+{
+    BatchSlot &q = b->sl[id];
+    emf_solver *s = q.s;
+    const int slot = q.slot;
+    const long long Tn = q.Tn, fixed_n0 = q.fixed_n0;
+    const long long n_stop = q.nmax < 0 ? 0 : (long long)floor(std::min(q.nmax, 1e15)) + 1;
+    const long long nlast = fixed_n0 >= 0 ? fixed_n0 : n_stop;
+    const long long nfac = nlast + 2 * Tn + 1;
+    // the solver's state as emf_solve sets it up (emopt/fdtd.py:1016-1018)
+    CHECK(build_samples(s));
+    PassTab th, te;
+    CHECK(refresh_tables(s, &th, &te));
+    CHECK(refresh_sources(s));
+    long long cap = std::min<long long>(nlast / Tn + 4, 1LL << 20);
+    if (cap > s->hist_cap) {
+        dfree(s->hist);
+        CHECK(dalloc(&s->hist, 3 * (size_t)cap));
+        s->hist_cap = (int)cap;
+    }
+    set_current(s, 0);
+    CHECK(reset_psi(s));
+    for (int c = 0; c < 3; ++c) {
+        HIPCHK(hipMemsetAsync(s->E[c], 0, s->n * sizeof(double), s->stream));
+        HIPCHK(hipMemsetAsync(s->H[c], 0, s->n * sizeof(double), s->stream));
+    }
+    HIPCHK(hipMemsetAsync(s->conv, 0, sizeof(ConvState), s->stream));
+    s->nhist = 0;
+
+    // per-step factors, computed exactly as the single-solve launches do
+    std::vector<double> f((size_t)nfac * NFAC);
+    for (long long q = 0; q < nfac; ++q) {
+        const double t = (double)q * s->dt, tE = ((double)q + 0.5) * s->dt;
+        double *r = &f[(size_t)q * NFAC];
+        r[0] = sin(t); r[1] = cos(t); r[2] = env_at(s, t);
+        r[3] = sin(tE); r[4] = cos(tE); r[5] = env_at(s, tE);
+        const double h = t - 0.5 * s->dt;
+        r[6] = sin(h); r[7] = cos(h);
+    }
+    CHECK(dalloc(&q.fac, f.size()));
+    int rc = hipMemcpyAsync(q.fac, f.data(), f.size() * sizeof(double), hipMemcpyHostToDevice,
+                            s->stream) == hipSuccess ? EMF_OK : EMF_ERR_HIP;
+    if (rc == EMF_OK && hipStreamSynchronize(s->stream) != hipSuccess) rc = EMF_ERR_HIP;
+    if (rc != EMF_OK) { dfree(q.fac); EMF_FAIL(rc, "upload of the step factors failed"); }
+
+    BMember &B = b->hM[id];
+    B.A = make_args(s, 0, 0);
+    B.g = s->geo();
+    B.g.zc = b->zc;
+    B.g.order = 0;
+    B.blk = s->src_desc;
+    B.nsrc = (int)s->srcs.size();
+    src_union(s, B.sub);
+    B.ntx = (s->Nx + PX - 1) / PX;
+    B.nty = (s->Ny + BTY - 1) / BTY;
+    B.ntz = (s->Nz + b->zc - 1) / b->zc;
+    B.fac = q.fac;
+    B.nfac = nfac;
+    B.res = reinterpret_cast<double *>(s->res[slot][0]);
+    B.n = s->n;
+    B.n_stop = n_stop;
+    B.fixed_n0 = fixed_n0;
+    B.Tn = Tn;
+    B.amp_rtol = q.rtol;
+    B.phi_rtol = sqrt(q.rtol);
+    B.dt = s->dt;
+    B.samples = s->samples;
+    B.nsamples = s->nsamples;
+    B.hist_cap = s->hist_cap;
+    B.conv = s->conv;
+    B.hist = s->hist;
+
+    BState st{};
+    st.mode = BM_STEP;
+    st.phase = BP_CONV;
+    if (nlast == 0) {                    // no steps before the t0 snapshot
+        st.mode = BM_CAP0;
+        st.phase = BP_RUN1;
+        st.status = fixed_n0 >= 0 ? 2 : 1;
+    }
+    // the batch's kernels may still be reading M/S/T: wait for them
+    CHECK(batch_sync(b));
+    HIPCHK(hipMemcpyAsync(&b->M[id], &B, sizeof(BMember), hipMemcpyHostToDevice, b->stream));
+    HIPCHK(hipMemcpyAsync(&b->S[id], &st, sizeof(BState), hipMemcpyHostToDevice, b->stream));
+    HIPCHK(hipStreamSynchronize(b->stream));   // B and st are locals
+    q.tiled = true;
+    return EMF_OK;
+}
+
+// The resident solve of member `id` (emf_solve's loop on its own stream).  The
+// handle refuses every other call while it is a member, so its lock is free.
+int batch_resident(emf_batch *b, int id, SolveRun &run)
+{
+    BatchSlot &q = b->sl[id];
+    HIPCHK(hipSetDevice(b->dev));
+    CHECK(solve_prepare(q.s, q.nmax, q.Tn));
+    CHECK(solve_any(q.s, q.slot, q.rtol, q.nmax, q.Tn, q.fixed_n0, run));
+    q.info.n0 = run.n0;
+    q.info.Tn = q.Tn;
+    q.info.steps = run.n0 + 2 * q.Tn;
+    q.info.status = run.status;
+    q.info.nchecks = run.nchecks;
+    q.info.a_change = run.a_change;
+    q.info.phi_change = run.phi_change;
+    q.info.seconds =
+        std::chrono::duration<double>(std::chrono::steady_clock::now() - q.t_add).count();
+    return EMF_OK;
 }
 
 }  // namespace
@@ -338,96 +457,34 @@ int emf_batch_add(emf_batch *b, emf_solver *s, int slot, double rtol, double nma
     const long long nfac = nlast + 2 * Tn + 1;
     if (nfac > (1LL << 22)) EMF_FAIL(EMF_ERR_ARG, "step limit %lld too large for a batch", nlast);
 
-    // the solver's state as emf_solve sets it up (emopt/fdtd.py:1016-1018)
     CHECK(ensure_slot(s, slot));
-    CHECK(build_samples(s));
-    PassTab th, te;
-    CHECK(refresh_tables(s, &th, &te));
-    CHECK(refresh_sources(s));
-    long long cap = std::min<long long>(nlast / Tn + 4, 1LL << 20);
-    if (cap > s->hist_cap) {
-        dfree(s->hist);
-        CHECK(dalloc(&s->hist, 3 * (size_t)cap));
-        s->hist_cap = (int)cap;
-    }
-    set_current(s, 0);
-    CHECK(reset_psi(s));
-    for (int c = 0; c < 3; ++c) {
-        HIPCHK(hipMemsetAsync(s->E[c], 0, s->n * sizeof(double), s->stream));
-        HIPCHK(hipMemsetAsync(s->H[c], 0, s->n * sizeof(double), s->stream));
-    }
-    HIPCHK(hipMemsetAsync(s->conv, 0, sizeof(ConvState), s->stream));
-    s->nhist = 0;
-
-    // per-step factors, computed exactly as the single-solve launches do
-    std::vector<double> f((size_t)nfac * NFAC);
-    for (long long q = 0; q < nfac; ++q) {
-        const double t = (double)q * s->dt, tE = ((double)q + 0.5) * s->dt;
-        double *r = &f[(size_t)q * NFAC];
-        r[0] = sin(t); r[1] = cos(t); r[2] = env_at(s, t);
-        r[3] = sin(tE); r[4] = cos(tE); r[5] = env_at(s, tE);
-        const double h = t - 0.5 * s->dt;
-        r[6] = sin(h); r[7] = cos(h);
-    }
+    ResPlan plan;
+    int ncu = 0;
+    CHECK(res_cus(s->dev, &ncu));
     BatchSlot &q = b->sl[id];
-    CHECK(dalloc(&q.fac, f.size()));
-    int rc = hipMemcpyAsync(q.fac, f.data(), f.size() * sizeof(double), hipMemcpyHostToDevice,
-                            s->stream) == hipSuccess ? EMF_OK : EMF_ERR_HIP;
-    if (rc == EMF_OK && hipStreamSynchronize(s->stream) != hipSuccess) rc = EMF_ERR_HIP;
-    if (rc != EMF_OK) { dfree(q.fac); EMF_FAIL(rc, "upload of the step factors failed"); }
-
-    BMember &B = b->hM[id];
-    B.A = make_args(s, 0, 0);
-    B.g = s->geo();
-    B.g.zc = b->zc;
-    B.g.order = 0;
-    B.blk = s->src_desc;
-    B.nsrc = (int)s->srcs.size();
-    src_union(s, B.sub);
-    B.ntx = (s->Nx + PX - 1) / PX;
-    B.nty = (s->Ny + BTY - 1) / BTY;
-    B.ntz = (s->Nz + b->zc - 1) / b->zc;
-    B.fac = q.fac;
-    B.nfac = nfac;
-    B.res = reinterpret_cast<double *>(s->res[slot][0]);
-    B.n = s->n;
-    B.n_stop = n_stop;
-    B.fixed_n0 = fixed_n0;
-    B.Tn = Tn;
-    B.amp_rtol = rtol;
-    B.phi_rtol = sqrt(rtol);
-    B.dt = s->dt;
-    B.samples = s->samples;
-    B.nsamples = s->nsamples;
-    B.hist_cap = s->hist_cap;
-    B.conv = s->conv;
-    B.hist = s->hist;
-
-    BState st{};
-    st.mode = BM_STEP;
-    st.phase = BP_CONV;
-    if (nlast == 0) {                    // no steps before the t0 snapshot
-        st.mode = BM_CAP0;
-        st.phase = BP_RUN1;
-        st.status = fixed_n0 >= 0 ? 2 : 1;
-    }
-    // the batch's kernels may still be reading M/S/T: wait for them
-    CHECK(batch_sync(b));
-    HIPCHK(hipMemcpyAsync(&b->M[id], &B, sizeof(BMember), hipMemcpyHostToDevice, b->stream));
-    HIPCHK(hipMemcpyAsync(&b->S[id], &st, sizeof(BState), hipMemcpyHostToDevice, b->stream));
     q.s = s;
-    s->in_batch = b;
     q.slot = slot;
-    q.finished = false;
+    q.finished = q.tiled = false;
     q.info = emf_solve_info{};
     q.t_add = std::chrono::steady_clock::now();
-    q.seq = b->next_seq++;
-    rc = batch_upload_table(b);           // synchronises the stream (B, st are locals)
+    q.rtol = rtol; q.nmax = nmax; q.Tn = Tn; q.fixed_n0 = fixed_n0;
+    // a member that fits on chip waits for its own resident solve (emf_batch_run)
+    const int rc = resident_plan(s, ncu, plan) ? solve_prepare(s, nmax, Tn) : batch_tile(b, id);
     if (rc != EMF_OK) {
-        q.s = nullptr;
-        s->in_batch = nullptr;
         dfree(q.fac);
+        q = BatchSlot{};
         return rc;
+    }
+    s->in_batch = b;
+    q.seq = b->next_seq++;
+    if (q.tiled) {
+        const int rt = batch_upload_table(b);
+        if (rt != EMF_OK) {
+            s->in_batch = nullptr;
+            dfree(q.fac);
+            q = BatchSlot{};
+            return rt;
+        }
     }
     *member = id;
     return EMF_OK;
@@ -443,7 +500,49 @@ int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished)
         for (auto &q : b->sl) r += q.s && !q.finished;
         return r;
     };
-    if (running() > 0) {
+    // members that fit on chip: each its own resident solve, a few at once where
+    // they leave CUs idle (the gate admits as many boxes as the device has CUs),
+    // and so that one's snapshots and host work overlap another's steps.  A run
+    // of a given number of replays steps them with the others instead.
+    std::vector<int> own;
+    for (int m = 0; m < BATCH_MAX; ++m)
+        if (b->sl[m].s && !b->sl[m].finished && !b->sl[m].tiled) own.push_back(m);
+    std::sort(own.begin(), own.end(), [&](int x, int y) { return b->sl[x].seq < b->sl[y].seq; });
+    if (until == 0 && !own.empty()) {
+        for (int m : own) {
+            std::lock_guard<std::mutex> lks(b->sl[m].s->mtx);
+            CHECK(batch_tile(b, m));
+        }
+        CHECK(batch_sync(b));
+        CHECK(batch_upload_table(b));
+        own.clear();
+    }
+    if (until == 1 && own.size() > 1) own.resize(1);
+    if (!own.empty()) {
+        std::atomic<size_t> next{ 0 };
+        std::mutex em;
+        int rc = EMF_OK;
+        std::string msg;
+        auto work = [&] {
+            for (size_t q; (q = next++) < own.size();) {
+                SolveRun run;
+                const int r = batch_resident(b, own[q], run);
+                std::lock_guard<std::mutex> lk(em);
+                if (r == EMF_OK) { b->sl[own[q]].finished = true; ++nfin; }
+                else if (rc == EMF_OK) { rc = r; msg = g_err; }
+            }
+        };
+        std::vector<std::thread> pool;
+        try {
+            for (size_t t = 1; t < std::min<size_t>(own.size(), BATCH_OWN); ++t) pool.emplace_back(work);
+        } catch (const std::system_error &) {
+            // no more threads: those there are (this one at least) take all members
+        }
+        work();
+        for (auto &t : pool) t.join();
+        if (rc != EMF_OK) EMF_FAIL(rc, "%s", msg.c_str());
+    }
+    if (running() > 0 && !(until == 1 && nfin > 0)) {
         CHECK(batch_graph(b));
         // a replay in flight: its lane, snapshot slot, group and end event
         struct Pend { int lane, r, g; hipEvent_t ev; };

@@ -22,6 +22,8 @@
 #include <condition_variable>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -1329,6 +1331,55 @@ int solve_run(emf_solver *s, int slot, double rtol, double nmax, long long Tn, l
     return EMF_OK;
 }
 
+
+// The device state of a solve loop: sample points and check history.
+int solve_prepare(emf_solver *s, double nmax, long long Tn)
+{
+    CHECK(build_samples(s));
+    if (fused(s)) CHECK(ensure_alt(s));
+    long long cap = (Tn > 0 ? (long long)(std::min(std::max(nmax, 0.0), 1e15) / (double)Tn) : 0) + 4;
+    cap = std::min<long long>(cap, 1LL << 20);
+    if (cap > s->hist_cap) {
+        dfree(s->hist);
+        CHECK(dalloc(&s->hist, 3 * (size_t)cap));
+        s->hist_cap = (int)cap;
+    }
+    return EMF_OK;
+}
+
+// solve_run with resident steps where the grid fits, else (or where they
+// stalled) with the step kernels; the history length and the final status.
+int solve_any(emf_solver *s, int slot, double rtol, double nmax, long long Tn, long long fixed_n0,
+              SolveRun &run)
+{
+    ResPlan plan;
+    int ncu = 0;
+    CHECK(res_cus(s->dev, &ncu));
+    if (resident_plan(s, ncu, plan)) {
+        ResHold hold;
+        hold.take(g_res_gate[s->dev], plan.boxes());
+        const int rc = solve_run(s, slot, rtol, nmax, Tn, fixed_n0, &plan, run);
+        if (rc != EMF_OK || run.stalled) (void)hipStreamSynchronize(s->stream);
+        hold.give();
+        CHECK(rc);
+        if (run.stalled) {
+            // the work-groups of a launch did not run together: from the start with the passes
+            s->res_off = true;
+            s->res_halo_clean = false;
+            CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
+        }
+    } else {
+        CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
+    }
+    s->nhist = std::min(run.nchecks, s->hist_cap);
+    // the loop runs on past non-finite samples (emopt/fdtd.py:1050-1052,
+    // 1137-1138) and stops at Nmax: say so when the last check saw them
+    if (run.status == 1 && run.nchecks > 0 &&
+        !(std::isfinite(run.a_change) && std::isfinite(run.phi_change)))
+        run.status = 3;
+    return EMF_OK;
+}
+
 }  // namespace
 
 // ---- allocation-free gradient assembly ----------------------------------
@@ -1894,43 +1945,11 @@ int emf_solve(emf_solver *s, int slot, double rtol, double nmax, int64_t Tn, int
     if (Tn < 0) EMF_FAIL(EMF_ERR_ARG, "Tn must be >= 0");
     CHECK(check_ready(s));
     CHECK(ensure_slot(s, slot));
-    CHECK(build_samples(s));
-    if (fused(s)) CHECK(ensure_alt(s));
-    long long cap = (Tn > 0 ? (long long)(std::min(std::max(nmax, 0.0), 1e15) / (double)Tn) : 0) + 4;
-    cap = std::min<long long>(cap, 1LL << 20);
-    if (cap > s->hist_cap) {
-        dfree(s->hist);
-        CHECK(dalloc(&s->hist, 3 * (size_t)cap));
-        s->hist_cap = (int)cap;
-    }
+    CHECK(solve_prepare(s, nmax, Tn));
     auto t_start = std::chrono::steady_clock::now();
-    ResPlan plan;
-    int ncu = 0;
-    CHECK(res_cus(s->dev, &ncu));
     SolveRun run;
-    if (resident_plan(s, ncu, plan)) {
-        ResHold hold;
-        hold.take(g_res_gate[s->dev], plan.boxes());
-        const int rc = solve_run(s, slot, rtol, nmax, Tn, fixed_n0, &plan, run);
-        if (rc != EMF_OK || run.stalled) (void)hipStreamSynchronize(s->stream);
-        hold.give();
-        CHECK(rc);
-        if (run.stalled) {
-            // the work-groups of a launch did not run together: from the start with the passes
-            s->res_off = true;
-            s->res_halo_clean = false;
-            CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
-        }
-    } else {
-        CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
-    }
+    CHECK(solve_any(s, slot, rtol, nmax, Tn, fixed_n0, run));
     auto t_end = std::chrono::steady_clock::now();
-    s->nhist = std::min(run.nchecks, s->hist_cap);
-    // the loop runs on past non-finite samples (emopt/fdtd.py:1050-1052,
-    // 1137-1138) and stops at Nmax: say so when the last check saw them
-    if (run.status == 1 && run.nchecks > 0 &&
-        !(std::isfinite(run.a_change) && std::isfinite(run.phi_change)))
-        run.status = 3;
     if (info) {
         info->n0 = run.n0;
         info->Tn = Tn;
