@@ -721,11 +721,13 @@ class FDTD(MaxwellSolver):
         the entry point that allocates no device memory (up to ~1 M
         entries)."""
         pidx = np.asarray(pidx, dtype=np.int32)
-        order = np.argsort(pidx, kind="stable")
-        pidx = np.ascontiguousarray(pidx[order])
-        comp = np.ascontiguousarray(np.asarray(comp, dtype=np.int32)[order])
-        cell = np.ascontiguousarray(np.asarray(cell, dtype=np.int64)[order])
-        deps = c128(np.asarray(deps, dtype=np.complex128)[order])
+        comp, cell = np.asarray(comp, dtype=np.int32), np.asarray(cell, dtype=np.int64)
+        deps = np.asarray(deps, dtype=np.complex128)
+        if np.any(pidx[1:] < pidx[:-1]):       # group by parameter
+            order = np.argsort(pidx, kind="stable")
+            pidx, comp, cell, deps = pidx[order], comp[order], cell[order], deps[order]
+        pidx, comp, cell = (np.ascontiguousarray(a) for a in (pidx, comp, cell))
+        deps = c128(deps)
         grad = np.zeros(int(nparam))
         fn = self._lib.emf_grad_assemble_noalloc if noalloc else self._lib.emf_grad_assemble
         fn(self._h, len(pidx), ptr(pidx), ptr(comp), ptr(cell), ptr(deps), int(nparam),
