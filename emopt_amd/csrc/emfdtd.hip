@@ -24,7 +24,6 @@
 #include <string>
 #include <system_error>
 #include <thread>
-#include <unordered_map>
 #include <vector>
 
 #include "../../include/emfdtd.h"
@@ -428,74 +427,63 @@ int refresh_coeffs(emf_solver *s)
     return EMF_OK;
 }
 
-// Index of distinct real eps triples, built on the host from the arrays
-// being uploaded.  Runs of equal cells along x are the common case, so the
-// previous cell's triple is checked before the hash map.
-struct EpsKey {
-    uint64_t a, b, c;
-    bool operator==(const EpsKey &o) const { return a == o.a && b == o.b && c == o.c; }
-};
-struct EpsKeyHash {
-    size_t operator()(const EpsKey &k) const
-    {
-        uint64_t h = k.a * 0x9E3779B97F4A7C15ULL;
-        h ^= k.b + 0x9E3779B97F4A7C15ULL + (h << 6) + (h >> 2);
-        h ^= k.c + 0x9E3779B97F4A7C15ULL + (h << 6) + (h >> 2);
-        return (size_t)h;
-    }
-};
-
-int build_coeff_index(emf_solver *s, const double *ex, const double *ey, const double *ez)
+// Index of the distinct real eps triples of the device's eps arrays
+// (k_idx_find): off (and the E pass on the full coefficients) with more than
+// IDX_LIMIT of them or with cells past the table's 32-bit numbers.
+int build_coeff_index(emf_solver *s)
 {
     dfree(s->cidx); dfree(s->ctabE); dfree(s->ctabB);
     s->cidx_valid = false;
     s->ctab_n = 0;
-    const long long n = s->n, limit = 1LL << 20;
-    std::unordered_map<EpsKey, uint32_t, EpsKeyHash> map;
-    std::vector<double> tab;
-    std::vector<uint32_t> idx((size_t)n);
-    EpsKey last{ ~0ULL, ~0ULL, ~0ULL };
-    uint32_t last_i = 0;
-    for (long long g = 0; g < n; ++g) {
-        EpsKey k;
-        memcpy(&k.a, &ex[2 * g], 8); memcpy(&k.b, &ey[2 * g], 8); memcpy(&k.c, &ez[2 * g], 8);
-        if (!(k == last)) {
-            auto it = map.find(k);
-            if (it == map.end()) {
-                if ((long long)map.size() >= limit) return EMF_OK;   // too many: stay off
-                last_i = (uint32_t)map.size();
-                map.emplace(k, last_i);
-                tab.push_back(ex[2 * g]); tab.push_back(ey[2 * g]); tab.push_back(ez[2 * g]);
-            } else {
-                last_i = it->second;
-            }
-            last = k;
+    const long long n = s->n;
+    if (n >= (long long)IDX_EMPTY) return EMF_OK;
+    unsigned slots = 1024;
+    while (slots < 4u * IDX_LIMIT && slots < 4ULL * (unsigned long long)n) slots *= 2;
+    unsigned *tmp = nullptr;           // slots, two counters, a slot per cell
+    if (dalloc(&tmp, (size_t)slots + 2 + (size_t)n) != EMF_OK) return EMF_OK;   // no room: off
+    unsigned *const head = tmp + slots, *const slot = head + 2;
+    unsigned cnt = 0;
+    int rc = EMF_OK;
+    auto ok = [&](hipError_t e) {
+        if (rc == EMF_OK && e != hipSuccess) {
+            set_err("coefficient index failed: %s", hipGetErrorString(e));
+            rc = EMF_ERR_HIP;
         }
-        idx[(size_t)g] = last_i;
+        return rc == EMF_OK;
+    };
+    hipLaunchKernelGGL(k_fill_u32, dim3(grid1d(slots, 256)), dim3(256), 0, s->stream, tmp,
+                       (long long)slots, IDX_EMPTY);
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s->stream, head, 2LL, 0u);
+    hipLaunchKernelGGL(k_idx_find, dim3(grid1d(n, 256)), dim3(256), 0, s->stream, s->eps[0],
+                       s->eps[1], s->eps[2], n, tmp, slots - 1, head, slot);
+    if (ok(hipGetLastError()) &&
+        ok(hipMemcpyAsync(&cnt, head, sizeof(cnt), hipMemcpyDeviceToHost, s->stream)) &&
+        ok(hipStreamSynchronize(s->stream)) && cnt <= (unsigned)IDX_LIMIT) {
+        uint16_t *d16 = nullptr;
+        uint32_t *d32 = nullptr;
+        rc = dalloc(&s->ctabE, 3 * (size_t)cnt);
+        if (rc == EMF_OK) rc = dalloc(&s->ctabB, 4 * (size_t)cnt);
+        if (rc == EMF_OK)   // the E pass reads aligned dwords
+            rc = cnt <= 65535 ? dalloc(&d16, (size_t)n + 2) : dalloc(&d32, (size_t)n);
+        s->cidx = d16 ? (void *)d16 : (void *)d32;
+        if (rc == EMF_OK) {
+            hipLaunchKernelGGL(k_idx_number, dim3(grid1d(slots, 256)), dim3(256), 0, s->stream,
+                               s->eps[0], s->eps[1], s->eps[2], tmp, slots, head + 1, s->ctabE);
+            if (d16)
+                hipLaunchKernelGGL(k_idx_write<uint16_t>, dim3(grid1d(n, 256)), dim3(256), 0,
+                                   s->stream, slot, tmp, n, d16);
+            else
+                hipLaunchKernelGGL(k_idx_write<uint32_t>, dim3(grid1d(n, 256)), dim3(256), 0,
+                                   s->stream, slot, tmp, n, d32);
+            if (ok(hipGetLastError()) && ok(hipStreamSynchronize(s->stream))) {
+                s->ctab_n = cnt;
+                s->cidx_valid = true;
+            }
+        }
     }
-    const long long nt = (long long)map.size();
-    CHECK(dalloc(&s->ctabE, 3 * (size_t)nt));
-    CHECK(dalloc(&s->ctabB, 4 * (size_t)nt));
-    HIPCHK(hipMemcpyAsync(s->ctabE, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice,
-                          s->stream));
-    if (nt <= 65535) {
-        std::vector<uint16_t> i16((size_t)n);
-        for (long long g = 0; g < n; ++g) i16[(size_t)g] = (uint16_t)idx[(size_t)g];
-        uint16_t *d = nullptr;
-        CHECK(dalloc(&d, (size_t)n + 2));   // the E pass reads aligned dwords
-        s->cidx = d;
-        HIPCHK(hipMemcpyAsync(d, i16.data(), n * sizeof(uint16_t), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-    } else {
-        uint32_t *d = nullptr;
-        CHECK(dalloc(&d, (size_t)n));
-        s->cidx = d;
-        HIPCHK(hipMemcpyAsync(d, idx.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-    }
-    s->ctab_n = nt;
-    s->cidx_valid = true;
-    return EMF_OK;
+    (void)hipStreamSynchronize(s->stream);
+    dfree(tmp);
+    return rc;
 }
 
 // CPML tables of compute_pml_params (src/fdtd.cpp:950-1181) into one device
@@ -1642,7 +1630,7 @@ int emf_set_mat_arrays(emf_solver *s, const double *ex, const double *ey, const 
                                   s->stream));
         }
     HIPCHK(hipStreamSynchronize(s->stream));
-    if (s->compress) CHECK(build_coeff_index(s, ex, ey, ez));
+    if (s->compress) CHECK(build_coeff_index(s));
     s->mat_set = true;
     s->coef_dirty = true;
     return EMF_OK;
@@ -2815,105 +2803,193 @@ int emf_set_h_shape(emf_solver *s, int tyg, int zc)
     return EMF_OK;
 }
 
+namespace {
+
+static_assert(sizeof(emf_prim) == sizeof(MatPrim), "emf_prim and MatPrim layouts differ");
+
+// The primitives of a structured material as given, checked.
+struct MatIn {
+    const emf_prim *prims;
+    int nprims;
+    const double *vx, *vy;
+    int nverts;
+    double dx, dy, dz;
+    int ss;
+    double bg_re, bg_im;
+};
+
+int mat_check(const MatIn &m)
+{
+    if (m.nprims < 0 || (m.nprims > 0 && !m.prims) || m.nverts < 0 || m.ss < 0 || m.ss > 64 ||
+        !(m.dx > 0) || !(m.dy > 0) || !(m.dz > 0))
+        EMF_FAIL(EMF_ERR_ARG, "bad arguments");
+    for (int q = 0; q < m.nprims; ++q) {
+        const emf_prim &p = m.prims[q];
+        if (p.kind < 0 || p.kind > 2) EMF_FAIL(EMF_ERR_ARG, "primitive %d: unknown kind", q);
+        if (m.ss == 0 && p.kind == 1)
+            EMF_FAIL(EMF_ERR_ARG, "primitive %d: the exact overlap rule takes ellipses as polygons", q);
+        if (p.kind == 2 &&
+            (p.v0 < 0 || p.nv < 0 || (long long)p.v0 + p.nv > m.nverts || !m.vx || !m.vy))
+            EMF_FAIL(EMF_ERR_ARG, "primitive %d: vertices out of range", q);
+    }
+    return EMF_OK;
+}
+
+// A box of cells and its offset within a cell (k, j, i ranges; sx, sy, sz).
+struct MatBox {
+    int k1, k2, j1, j2, i1, i2;
+    double sx, sy, sz;
+};
+
+// Samples the material on `nbox` boxes into device arrays out[q]: the in-plane
+// values of every box first, and only when no cell was refused the boxes
+// themselves, so that a refusal leaves them as they were.
+int mat_sample(const MatIn &m, const MatBox *box, double2 *const *out, int nbox, hipStream_t st)
+{
+    // z segments as the host sampler forms them: consecutive distinct primitive
+    // z bounds, skipped when no cell of the box overlaps them
+    std::vector<double> b;
+    for (int q = 0; q < m.nprims; ++q) {
+        if (!(m.prims[q].z2 > m.prims[q].z1)) continue;
+        b.push_back(m.prims[q].z1);
+        b.push_back(m.prims[q].z2);
+    }
+    std::sort(b.begin(), b.end());
+    b.erase(std::unique(b.begin(), b.end()), b.end());
+    struct Part { int nseg; size_t zab, off, v2; };
+    std::vector<Part> part(nbox);
+    std::vector<double> zab;
+    std::vector<int> off, sp;
+    size_t nv2 = 0;
+    for (int x = 0; x < nbox; ++x) {
+        const MatBox &B = box[x];
+        part[x].zab = zab.size();
+        part[x].off = off.size();
+        part[x].v2 = nv2;
+        off.push_back((int)sp.size());
+        for (size_t s = 0; s + 1 < b.size(); ++s) {
+            const double za = b[s], zb = b[s + 1];
+            bool used = false;
+            for (int i = B.i1; i < B.i2 && !used; ++i) {
+                const double zc = ((double)i + B.sz) * m.dz;
+                const double zlo = zc - m.dz / 2, zhi = zc + m.dz / 2;
+                used = std::max(std::min(zhi, zb) - std::max(zlo, za), 0.0) / m.dz > 0;
+            }
+            if (!used) continue;
+            zab.push_back(za);
+            zab.push_back(zb);
+            for (int q = 0; q < m.nprims; ++q)
+                if (m.prims[q].z2 > m.prims[q].z1 && m.prims[q].z1 <= za && m.prims[q].z2 >= zb)
+                    sp.push_back(q);
+            off.push_back((int)sp.size());
+        }
+        part[x].nseg = (int)(off.size() - part[x].off) - 1;
+        nv2 += (size_t)part[x].nseg * (B.j2 - B.j1) * (B.k2 - B.k1);
+    }
+    // one staging block: primitives, vertices, segment bounds, offsets, lists, error
+    const size_t o_vx = align_up(m.nprims * sizeof(MatPrim)), o_vy = align_up(o_vx + m.nverts * 8);
+    const size_t o_z = align_up(o_vy + m.nverts * 8), o_off = align_up(o_z + zab.size() * 8);
+    const size_t o_sp = align_up(o_off + off.size() * 4), o_err = align_up(o_sp + sp.size() * 4);
+    std::vector<unsigned char> h(o_err + sizeof(int), 0);
+    if (m.nprims) memcpy(&h[0], m.prims, m.nprims * sizeof(MatPrim));
+    if (m.nverts && m.vx) memcpy(&h[o_vx], m.vx, m.nverts * 8);
+    if (m.nverts && m.vy) memcpy(&h[o_vy], m.vy, m.nverts * 8);
+    if (!zab.empty()) memcpy(&h[o_z], zab.data(), zab.size() * 8);
+    memcpy(&h[o_off], off.data(), off.size() * 4);
+    if (!sp.empty()) memcpy(&h[o_sp], sp.data(), sp.size() * 4);
+    unsigned char *d = nullptr;
+    double2 *v2 = nullptr;
+    int rc = dalloc(&d, h.size());
+    if (rc == EMF_OK) rc = dalloc(&v2, nv2);
+    int cell_err = 0;
+    auto ok = [&](hipError_t e) { if (rc == EMF_OK && e != hipSuccess) rc = EMF_ERR_HIP; return rc == EMF_OK; };
+    if (rc == EMF_OK && ok(hipMemcpyAsync(d, h.data(), h.size(), hipMemcpyHostToDevice, st))) {
+        for (int x = 0; x < nbox; ++x) {
+            const MatBox &B = box[x];
+            const int nk = B.k2 - B.k1, nj = B.j2 - B.j1;
+            const long long nw = (long long)part[x].nseg * nj * nk;
+            if (nw > 0)
+                hipLaunchKernelGGL(k_mat_inplane, dim3(grid1d(nw, 64)), dim3(64), 0, st,
+                                   (const MatPrim *)d, (const double *)(d + o_vx),
+                                   (const double *)(d + o_vy), (const int *)(d + o_off) + part[x].off,
+                                   (const int *)(d + o_sp), part[x].nseg, B.k1, nk, B.j1, nj, B.sx,
+                                   B.sy, m.dx, m.dy, m.ss, m.bg_re, m.bg_im, v2 + part[x].v2,
+                                   (int *)(d + o_err));
+        }
+        ok(hipGetLastError());
+        if (nv2 > 0 && ok(hipMemcpyAsync(&cell_err, d + o_err, sizeof(int), hipMemcpyDeviceToHost, st)))
+            ok(hipStreamSynchronize(st));
+        for (int x = 0; x < nbox && rc == EMF_OK && !cell_err; ++x) {
+            const MatBox &B = box[x];
+            const int nk = B.k2 - B.k1, nj = B.j2 - B.j1, ni = B.i2 - B.i1;
+            hipLaunchKernelGGL(k_mat_combine, dim3(grid1d((long long)ni * nj * nk, 256)), dim3(256), 0,
+                               st, v2 + part[x].v2, (const double *)(d + o_z) + part[x].zab,
+                               part[x].nseg, B.i1, ni, nj, nk, B.sz, m.dz, m.bg_re, m.bg_im, out[x]);
+            ok(hipGetLastError());
+        }
+    }
+    ok(hipStreamSynchronize(st));     // h, d and v2 are done with
+    dfree(d); dfree(v2);
+    if (rc != EMF_OK) EMF_FAIL(rc, "material sampling failed");
+    if (cell_err)
+        EMF_FAIL(EMF_ERR_ARG, "a cell meets more than %d primitives or %d polygon edges "
+                 "(exact overlap rule)", MAT_MAXU, MAT_MAXE);
+    return EMF_OK;
+}
+
+}  // namespace
+
 int emf_sample_structured(int device, const emf_prim *prims, int nprims, const double *vx,
                           const double *vy, int nverts, double dx, double dy, double dz,
                           int supersample, double bg_re, double bg_im, int k1, int k2, int j1,
                           int j2, int i1, int i2, double sx, double sy, double sz, double *out)
 {
-    static_assert(sizeof(emf_prim) == sizeof(MatPrim), "emf_prim and MatPrim layouts differ");
-    if (!out || nprims < 0 || (nprims > 0 && !prims) || nverts < 0 || supersample < 0 ||
-        supersample > 64 || !(dx > 0) || !(dy > 0) || !(dz > 0) || k2 <= k1 || j2 <= j1 ||
-        i2 <= i1)
-        EMF_FAIL(EMF_ERR_ARG, "bad arguments");
-    for (int q = 0; q < nprims; ++q) {
-        const emf_prim &p = prims[q];
-        if (p.kind < 0 || p.kind > 2) EMF_FAIL(EMF_ERR_ARG, "primitive %d: unknown kind", q);
-        if (supersample == 0 && p.kind == 1)
-            EMF_FAIL(EMF_ERR_ARG, "primitive %d: the exact overlap rule takes ellipses as polygons", q);
-        if (p.kind == 2 && (p.v0 < 0 || p.nv < 0 || (long long)p.v0 + p.nv > nverts || !vx || !vy))
-            EMF_FAIL(EMF_ERR_ARG, "primitive %d: vertices out of range", q);
-    }
-    const int nk = k2 - k1, nj = j2 - j1, ni = i2 - i1;
-    const long long ncell = (long long)ni * nj * nk;
-    // z segments as the host sampler forms them: consecutive distinct primitive
-    // z bounds, skipped when no cell of the box overlaps them
-    std::vector<double> b;
-    for (int q = 0; q < nprims; ++q) {
-        if (!(prims[q].z2 > prims[q].z1)) continue;
-        b.push_back(prims[q].z1);
-        b.push_back(prims[q].z2);
-    }
-    std::sort(b.begin(), b.end());
-    b.erase(std::unique(b.begin(), b.end()), b.end());
-    std::vector<double> zab;
-    std::vector<int> off(1, 0), sp;
-    for (size_t s = 0; s + 1 < b.size(); ++s) {
-        const double za = b[s], zb = b[s + 1];
-        bool used = false;
-        for (int i = i1; i < i2 && !used; ++i) {
-            const double zc = ((double)i + sz) * dz;
-            const double zlo = zc - dz / 2, zhi = zc + dz / 2;
-            used = std::max(std::min(zhi, zb) - std::max(zlo, za), 0.0) / dz > 0;
-        }
-        if (!used) continue;
-        zab.push_back(za);
-        zab.push_back(zb);
-        for (int q = 0; q < nprims; ++q)
-            if (prims[q].z2 > prims[q].z1 && prims[q].z1 <= za && prims[q].z2 >= zb) sp.push_back(q);
-        off.push_back((int)sp.size());
-    }
-    const int nseg = (int)zab.size() / 2;
+    if (!out || k2 <= k1 || j2 <= j1 || i2 <= i1) EMF_FAIL(EMF_ERR_ARG, "bad arguments");
+    const MatIn m{ prims, nprims, vx, vy, nverts, dx, dy, dz, supersample, bg_re, bg_im };
+    CHECK(mat_check(m));
+    const long long ncell = (long long)(i2 - i1) * (j2 - j1) * (k2 - k1);
     HIPCHK(hipSetDevice(device));
     hipStream_t st;
     HIPCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    MatPrim *dp = nullptr;
-    double *dvx = nullptr, *dvy = nullptr, *dz_ab = nullptr;
-    int *doff = nullptr, *dsp = nullptr, *derr = nullptr;
-    double2 *v2 = nullptr, *dout = nullptr;
-    int rc = EMF_OK;
-    auto ok = [&](int r) { if (rc == EMF_OK && r != EMF_OK) rc = r; return rc == EMF_OK; };
-    if (ok(dalloc(&dout, (size_t)ncell)) && nseg > 0 && ok(dalloc(&dp, (size_t)nprims)) &&
-        ok(dalloc(&doff, off.size())) && ok(dalloc(&dsp, std::max<size_t>(1, sp.size()))) &&
-        ok(dalloc(&dz_ab, zab.size())) && ok(dalloc(&v2, (size_t)nseg * nj * nk)) &&
-        ok(dalloc(&derr, 1)) &&
-        (nverts == 0 || (ok(dalloc(&dvx, (size_t)nverts)) && ok(dalloc(&dvy, (size_t)nverts))))) {
-        if (hipMemcpyAsync(dp, prims, nprims * sizeof(MatPrim), hipMemcpyHostToDevice, st) != hipSuccess ||
-            hipMemcpyAsync(doff, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice, st) != hipSuccess ||
-            (!sp.empty() && hipMemcpyAsync(dsp, sp.data(), sp.size() * sizeof(int), hipMemcpyHostToDevice, st) != hipSuccess) ||
-            hipMemcpyAsync(dz_ab, zab.data(), zab.size() * sizeof(double), hipMemcpyHostToDevice, st) != hipSuccess ||
-            (nverts > 0 && (hipMemcpyAsync(dvx, vx, nverts * sizeof(double), hipMemcpyHostToDevice, st) != hipSuccess ||
-                            hipMemcpyAsync(dvy, vy, nverts * sizeof(double), hipMemcpyHostToDevice, st) != hipSuccess)))
+    double2 *dout = nullptr;
+    const MatBox box{ k1, k2, j1, j2, i1, i2, sx, sy, sz };
+    int rc = dalloc(&dout, (size_t)ncell);
+    if (rc == EMF_OK) rc = mat_sample(m, &box, &dout, 1, st);
+    if (rc == EMF_OK) {
+        if (device < HOST_DEVICES) {
+            rc = download(device, st, out, dout, (size_t)ncell * sizeof(double2));
+        } else if (hipMemcpyAsync(out, dout, (size_t)ncell * sizeof(double2), hipMemcpyDeviceToHost,
+                                  st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
+            set_err("download failed");
             rc = EMF_ERR_HIP;
-        if (rc == EMF_OK && hipMemsetAsync(derr, 0, sizeof(int), st) != hipSuccess) rc = EMF_ERR_HIP;
-        if (rc == EMF_OK) {
-            const long long nv2 = (long long)nseg * nj * nk;
-            hipLaunchKernelGGL(k_mat_inplane, dim3(grid1d(nv2, 256)), dim3(256), 0, st, dp, dvx, dvy,
-                               doff, dsp, nseg, k1, nk, j1, nj, sx, sy, dx, dy, supersample, bg_re,
-                               bg_im, v2, derr);
-            if (hipGetLastError() != hipSuccess) rc = EMF_ERR_HIP;
         }
     }
-    int cell_err = 0;
-    if (rc == EMF_OK && derr &&
-        (hipMemcpyAsync(&cell_err, derr, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess ||
-         hipStreamSynchronize(st) != hipSuccess))
-        rc = EMF_ERR_HIP;
-    if (rc == EMF_OK) {
-        hipLaunchKernelGGL(k_mat_combine, dim3(grid1d(ncell, 256)), dim3(256), 0, st, v2, dz_ab, nseg,
-                           i1, ni, nj, nk, sz, dz, bg_re, bg_im, dout);
-        if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(out, dout, (size_t)ncell * sizeof(double2), hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess)
-            rc = EMF_ERR_HIP;
-    }
     (void)hipStreamSynchronize(st);
-    dfree(dp); dfree(dvx); dfree(dvy); dfree(dz_ab); dfree(doff); dfree(dsp); dfree(v2); dfree(dout);
-    dfree(derr);
+    dfree(dout);
     (void)hipStreamDestroy(st);
-    if (rc != EMF_OK) EMF_FAIL(rc, "material sampling failed");
-    if (cell_err)
-        EMF_FAIL(EMF_ERR_ARG, "a cell meets more than %d primitives or %d polygon edges "
-                 "(exact overlap rule)", MAT_MAXU, MAT_MAXE);
+    return rc;
+}
+
+int emf_build_structured(emf_solver *s, const emf_prim *prims, int nprims, const double *vx,
+                         const double *vy, int nverts, double dx, double dy, double dz,
+                         int supersample, double bg_re, double bg_im, const double *shifts,
+                         double mu_re)
+{
+    LOCK(s);
+    if (!shifts) EMF_FAIL(EMF_ERR_ARG, "null argument");
+    const MatIn m{ prims, nprims, vx, vy, nverts, dx, dy, dz, supersample, bg_re, bg_im };
+    CHECK(mat_check(m));
+    CHECK(ensure_fields(s));
+    MatBox box[3];
+    for (int c = 0; c < 3; ++c)
+        box[c] = MatBox{ 0, s->Nx, 0, s->Ny, 0, s->Nz, shifts[3 * c], shifts[3 * c + 1], shifts[3 * c + 2] };
+    CHECK(mat_sample(m, box, s->eps, 3, s->stream));
+    s->mu_uniform = true;
+    s->mu_re = mu_re;
+    s->coef_dirty = true;
+    s->cidx_valid = false;
+    s->mat_set = true;
+    if (s->compress) CHECK(build_coeff_index(s));
     return EMF_OK;
 }
 

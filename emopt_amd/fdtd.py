@@ -18,6 +18,7 @@ domain decomposition (PETSc DMDA, GhostComm) has no counterpart.
 """
 from __future__ import annotations
 
+import math
 import warnings
 from math import pi
 
@@ -26,7 +27,7 @@ import numpy as np
 from . import _lib
 from ._lib import SolveInfo, c128, ptr
 from .defs import FIELD_INDEX, FieldComponent
-from .grid import StructuredMaterial3D
+from .grid import ConstantMaterial3D, StructuredMaterial3D
 from .misc import DomainCoordinates
 from .simulation import MaxwellSolver
 
@@ -273,6 +274,12 @@ class FDTD(MaxwellSolver):
         (emopt/fdtd.py:842-880)."""
         if self._eps is None or self._mu is None:
             raise RuntimeError("set_materials(eps, mu) must be called before build()")
+        if self._samples_in_place():
+            self._eps.build_device(self._lib, self._h, self.YEE_SHIFTS[:3],
+                                   self._mu.material_value.real)
+            self._mu_uniform = True
+            self._mats_ready = True
+            return
         Nx, Ny, Nz = self._Nx, self._Ny, self._Nz
         arrs = []
         for q, (sx, sy, sz) in enumerate(self.YEE_SHIFTS):
@@ -281,6 +288,16 @@ class FDTD(MaxwellSolver):
             self._sample(m, 0, Nx, 0, Ny, 0, Nz, sx, sy, sz, arr=a)
             arrs.append(c128(a))
         self.set_material_arrays(arrs[:3], arrs[3:])
+
+    def _samples_in_place(self):
+        """Whether the GPU samples eps where the solver reads it: a structured
+        eps with the samplers of its class as they are, and one mu.  Anything
+        that replaces them is asked for its arrays instead."""
+        return (isinstance(self._eps, StructuredMaterial3D) and self._eps.stock_samplers()
+                and type(self._mu) is ConstantMaterial3D
+                and math.isfinite(self._mu.material_value.real)
+                and type(self)._sample is FDTD._sample
+                and type(self).set_material_arrays is FDTD.set_material_arrays)
 
     def _sample(self, m, k1, k2, j1, j2, i1, i2, sx, sy, sz, arr=None):
         """Material values of a box at one Yee offset: structured materials

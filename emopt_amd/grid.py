@@ -307,6 +307,9 @@ class Polygon(_Sampled):
 
 def _clip_to_box(xs, ys, box):
     """Sutherland-Hodgman clip of a polygon to an axis-aligned box."""
+    if len(xs) >= 3 and min(xs) >= box[0] and max(xs) <= box[1] and min(ys) >= box[2] \
+            and max(ys) <= box[3]:
+        return np.array(xs), np.array(ys)        # inside: as it is
     pts = list(zip(xs, ys))
     for axis, val, keep_above in ((0, box[0], True), (0, box[1], False),
                                   (1, box[2], True), (1, box[3], False)):
@@ -664,6 +667,22 @@ class StructuredMaterial3D(Material3D):
                                   k1, k2, j1, j2, i1, i2, sx, sy, sz, out.ctypes.data)
         return self._out(out, arr, reshape)
 
+    def stock_samplers(self):
+        """Whether get_values and get_values_device are this module's own."""
+        return all(getattr(getattr(self, f), "__func__", None) is fn
+                   for f, fn in _STOCK_SAMPLERS.items())
+
+    def build_device(self, lib, handle, shifts, mu):
+        """Sample eps at three in-cell offsets straight into a solver's arrays
+        (emf_build_structured), with the uniform mu `mu`."""
+        recs, vx, vy, nv = self.device_primitives()
+        sh = np.ascontiguousarray(shifts, dtype=np.double)
+        lib.emf_build_structured(handle, recs.ctypes.data, len(recs), vx.ctypes.data,
+                                 vy.ctypes.data, nv, self._dx, self._dy, self._dz,
+                                 0 if self.overlap == "exact" else int(self.supersample),
+                                 self.background.real, self.background.imag, sh.ctypes.data,
+                                 float(mu))
+
     def get_values(self, k1, k2, j1, j2, i1, i2, sx=0.0, sy=0.0, sz=0.0, arr=None, reshape=True):
         dx, dy, dz = self._dx, self._dy, self._dz
         xc = (np.arange(k1, k2) + sx) * dx
@@ -687,3 +706,7 @@ class StructuredMaterial3D(Material3D):
             covered += fz
         out += (1.0 - covered)[:, None, None] * self.background
         return self._out(out, arr, reshape)
+
+
+_STOCK_SAMPLERS = {"get_values": StructuredMaterial3D.get_values,
+                   "get_values_device": StructuredMaterial3D.get_values_device}

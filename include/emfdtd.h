@@ -462,6 +462,16 @@ EMF_API int emf_sample_structured(int device, const emf_prim *prims, int nprims,
                                   double bg_im, int k1, int k2, int j1, int j2, int i1, int i2,
                                   double sx, double sy, double sz, double *out);
 
+/* Materials of a solver from a structured eps (the primitives, as above) and a
+ * uniform mu: eps_x, eps_y, eps_z are sampled over the whole grid at the
+ * in-cell offsets shifts[3 c .. 3 c + 2] straight into the solver's arrays, with
+ * the values emf_sample_structured gives, in the place of emf_set_mat_arrays.
+ * A refused cell leaves the solver's materials as they were. */
+EMF_API int emf_build_structured(emf_solver *s, const emf_prim *prims, int nprims,
+                                 const double *vx, const double *vy, int nverts, double dx,
+                                 double dy, double dz, int supersample, double bg_re,
+                                 double bg_im, const double *shifts, double mu_re);
+
 typedef struct emf_batch emf_batch;
 
 EMF_API int emf_batch_new(int device, emf_batch **out);
