@@ -2908,13 +2908,18 @@ int mat_sample(const MatIn &m, const MatBox *box, double2 *const *out, int nbox,
             const MatBox &B = box[x];
             const int nk = B.k2 - B.k1, nj = B.j2 - B.j1;
             const long long nw = (long long)part[x].nseg * nj * nk;
-            if (nw > 0)
-                hipLaunchKernelGGL(k_mat_inplane, dim3(grid1d(nw, 64)), dim3(64), 0, st,
-                                   (const MatPrim *)d, (const double *)(d + o_vx),
-                                   (const double *)(d + o_vy), (const int *)(d + o_off) + part[x].off,
-                                   (const int *)(d + o_sp), part[x].nseg, B.k1, nk, B.j1, nj, B.sx,
-                                   B.sy, m.dx, m.dy, m.ss, m.bg_re, m.bg_im, v2 + part[x].v2,
+            const MatPrim *const dp = (const MatPrim *)d;
+            const double *const dvx = (const double *)(d + o_vx), *const dvy = (const double *)(d + o_vy);
+            const int *const doff = (const int *)(d + o_off) + part[x].off, *const dsp = (const int *)(d + o_sp);
+            if (nw > 0 && m.ss == 0)
+                hipLaunchKernelGGL(k_mat_exact, dim3((unsigned)std::min(nw, 1LL << 20)), dim3(64), 0, st,
+                                   dp, dvx, dvy, doff, dsp, part[x].nseg, B.k1, nk, B.j1, nj, B.sx,
+                                   B.sy, m.dx, m.dy, m.bg_re, m.bg_im, v2 + part[x].v2,
                                    (int *)(d + o_err));
+            else if (nw > 0)
+                hipLaunchKernelGGL(k_mat_inplane, dim3(grid1d(nw, 64)), dim3(64), 0, st, dp, dvx, dvy,
+                                   doff, dsp, part[x].nseg, B.k1, nk, B.j1, nj, B.sx, B.sy, m.dx,
+                                   m.dy, m.ss, m.bg_re, m.bg_im, v2 + part[x].v2);
         }
         ok(hipGetLastError());
         if (nv2 > 0 && ok(hipMemcpyAsync(&cell_err, d + o_err, sizeof(int), hipMemcpyDeviceToHost, st)))
