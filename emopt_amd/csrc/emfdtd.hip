@@ -164,6 +164,7 @@ struct emf_solver {
     int bc[3] = { '0', '0', '0' };
     int nconv = 10;
     int zc = 2;
+    bool zc_auto = true;           // zc not chosen by the caller
     int order = 3;                 // two-pass work-group order (pass_tile)
     int psi_stream = -1;           // streaming psi access: -1 by size, 0 off, 1 on
 
@@ -714,16 +715,34 @@ FusedArgs make_args(const emf_solver *s, int from, int to)
     return A;
 }
 
+// Whether what a step touches -- fields, coefficients and psi -- stays in the
+// 256 MB Infinity Cache from step to step (some of which other data takes).
+inline bool step_cached(const emf_solver *s)
+{
+    const bool idx = s->cidx_bytes != 0 && s->compress && s->cidx_valid && !s->ceps;
+    const double cell = 48.0 + (idx ? s->cidx_bytes : 24.0) + (s->ceps ? 24.0 : 0.0) +
+                        (s->mu_uniform ? 0.0 : 24.0);
+    return (double)s->n * cell + 16.0 * (double)s->psi_tot < 250e6;
+}
+
 // Whether the passes stream the psi arrays past the caches (non-temporal):
-// when a step's data -- fields, coefficients and psi -- exceeds the 256 MB
-// Infinity Cache, nothing of it survives to the next step and psi lines would
-// only displace the fields the next pass re-reads; a smaller solve keeps its
-// psi cached from step to step.  emf_set_streaming overrides.
+// when a step's data does not stay in the Infinity Cache, psi lines would only
+// displace the fields the next pass re-reads (400x200x120: 313 -> 299 us a
+// step); a smaller solve keeps its psi cached from step to step
+// (360x60x120: 90 -> 72 us without streaming).  emf_set_streaming overrides.
 inline bool stream_psi(const emf_solver *s)
 {
     if (s->psi_stream >= 0) return s->psi_stream == 1;
-    const double bytes = (double)s->n * 100.0 + 2.0 * 2.0 * 8.0 * (double)s->psi_tot;
-    return bytes > 256e6;
+    return !step_cached(s);
+}
+
+// Rows of a strip of the two passes (pass_tile), 0 for none: the grid's rows in
+// equal parts of at most 48.
+int pass_strip(const emf_solver *s)
+{
+    if (!step_cached(s)) return 0;
+    const int parts = (s->Ny + 47) / 48;
+    return ((s->Ny + parts - 1) / parts + 7) / 8 * 8;
 }
 
 // rows per work-group of the two passes (tyg of a fused kind may be 16)
@@ -742,10 +761,10 @@ int pass_ty(const emf_solver *s)
             hipLaunchKernelGGL(K, GR, BLK, 0, s->stream, __VA_ARGS__);                       \
     } while (0)
 
-dim3 pass_grid(const emf_solver *s)
+dim3 pass_grid(const emf_solver *s, const Geo &g)
 {
     const int ty = pass_ty(s);
-    return dim3((s->Nx + PX - 1) / PX, (s->Ny + ty - 1) / ty, (s->Nz + s->zc - 1) / s->zc);
+    return dim3((s->Nx + PX - 1) / PX, (s->Ny + ty - 1) / ty, (s->Nz + g.zc - 1) / g.zc);
 }
 
 // the H pass's work-group shape: its own when set, else the E pass's
@@ -755,7 +774,14 @@ int pass_ty_h(const emf_solver *s)
     return t == 1 || t == 2 || t == 8 ? t : 4;
 }
 
-int pass_zc_h(const emf_solver *s) { return s->zc_h > 0 ? s->zc_h : s->zc; }
+// Planes per work-group of the passes.  One where the step's data stays in the
+// Infinity Cache and tiles are strips, unless the caller chose: the planes next
+// to a tile's are in L2 anyway, and more work-groups hide more latency (us a
+// step, 2 -> 1: 173x101x67 with complex eps 44.2 -> 41.5, 360x60x120 70.8
+// -> 67.5, 200x100x100 63.2 -> 64.1); elsewhere 2 (400x200x120: 296, 303 with 1).
+int pass_zc(const emf_solver *s) { return s->zc_auto && pass_strip(s) > 0 ? 1 : s->zc; }
+
+int pass_zc_h(const emf_solver *s) { return s->zc_h > 0 ? s->zc_h : pass_zc(s); }
 
 template <bool MU, int OCC, bool NT>
 void launch_h_occ(const emf_solver *s, const FusedArgs &A, const Geo &g, const PassSrc &ps,
@@ -775,7 +801,7 @@ template <int CM, int OCC, int ZU, bool NT>
 void launch_e_zu(const emf_solver *s, const FusedArgs &A, const Geo &g, const PassSrc &ps,
                  const int *done)
 {
-    const dim3 gr = pass_grid(s);
+    const dim3 gr = pass_grid(s, g);
     switch (pass_ty(s)) {
     case 1: PASS_LAUNCH((k_pass_e<CM, 1, OCC, ZU, NT>), gr, dim3(PX, 1), A, g, ps, done); break;
     case 2: PASS_LAUNCH((k_pass_e<CM, 2, OCC, ZU, NT>), gr, dim3(PX, 2), A, g, ps, done); break;
@@ -789,9 +815,10 @@ template <int CM, int OCC, bool NT>
 void launch_e_occ(const emf_solver *s, const FusedArgs &A, const Geo &g, const PassSrc &ps,
                   const int *done)
 {
-    if (CM == CM_INDEX && s->zc <= 2) launch_e_zu<CM, OCC, 2, NT>(s, A, g, ps, done);
-    else if (CM == CM_INDEX && s->zc <= 4) launch_e_zu<CM, OCC, 4, NT>(s, A, g, ps, done);
-    else if (CM == CM_INDEX && s->zc <= 8) launch_e_zu<CM, OCC, 8, NT>(s, A, g, ps, done);
+    if (CM == CM_INDEX && g.zc <= 1) launch_e_zu<CM, OCC, 1, NT>(s, A, g, ps, done);
+    else if (CM == CM_INDEX && g.zc <= 2) launch_e_zu<CM, OCC, 2, NT>(s, A, g, ps, done);
+    else if (CM == CM_INDEX && g.zc <= 4) launch_e_zu<CM, OCC, 4, NT>(s, A, g, ps, done);
+    else if (CM == CM_INDEX && g.zc <= 8) launch_e_zu<CM, OCC, 8, NT>(s, A, g, ps, done);
     else launch_e_zu<CM, OCC, 0, NT>(s, A, g, ps, done);
 }
 
@@ -809,7 +836,7 @@ template <int CM, int ZU, bool NT>
 void launch_e_wide_zu(const emf_solver *s, const FusedArgs &A, const Geo &g, const PassSrc &ps,
                       const int *done)
 {
-    const dim3 gr((s->Nx + PX - 1) / PX, (s->Ny + 3) / 4, (s->Nz + s->zc - 1) / s->zc);
+    const dim3 gr((s->Nx + PX - 1) / PX, (s->Ny + 3) / 4, (s->Nz + g.zc - 1) / g.zc);
     PASS_LAUNCH((k_pass_e<CM, 4, 4, ZU, NT, true>), gr, dim3(PX, 4), A, g, ps, done);
 }
 
@@ -817,9 +844,9 @@ template <int CM, bool NT>
 void launch_e_wide(const emf_solver *s, const FusedArgs &A, const Geo &g, const PassSrc &ps,
                    const int *done)
 {
-    if (CM == CM_INDEX && s->zc <= 2) launch_e_wide_zu<CM, 2, NT>(s, A, g, ps, done);
-    else if (CM == CM_INDEX && s->zc <= 4) launch_e_wide_zu<CM, 4, NT>(s, A, g, ps, done);
-    else if (CM == CM_INDEX && s->zc <= 8) launch_e_wide_zu<CM, 8, NT>(s, A, g, ps, done);
+    if (CM == CM_INDEX && g.zc <= 2) launch_e_wide_zu<CM, 2, NT>(s, A, g, ps, done);
+    else if (CM == CM_INDEX && g.zc <= 4) launch_e_wide_zu<CM, 4, NT>(s, A, g, ps, done);
+    else if (CM == CM_INDEX && g.zc <= 8) launch_e_wide_zu<CM, 8, NT>(s, A, g, ps, done);
     else launch_e_wide_zu<CM, 0, NT>(s, A, g, ps, done);
 }
 
@@ -875,6 +902,7 @@ int launch_h(emf_solver *s, double t, const int *done)
     FusedArgs A = make_args(s, s->cur, s->cur);
     Geo g = s->geo();
     g.zc = pass_zc_h(s);
+    g.strip = pass_strip(s);
     if (s->mu_uniform) launch_h_t<false>(s, A, g, ps, done);
     else launch_h_t<true>(s, A, g, ps, done);
     HIPCHK(hipGetLastError());
@@ -890,6 +918,8 @@ int launch_e(emf_solver *s, double t, const int *done)
     PassSrc ps = pass_sources(s, 0, t);
     FusedArgs A = make_args(s, s->cur, s->cur);
     Geo g = s->geo();
+    g.zc = pass_zc(s);
+    g.strip = pass_strip(s);
     if (s->ceps) launch_e_t<CM_COMPLEX>(s, A, g, ps, done);
     else if (A.bI) launch_e_t<CM_INDEX>(s, A, g, ps, done);
     else launch_e_t<CM_REAL>(s, A, g, ps, done);
@@ -2759,6 +2789,7 @@ int emf_set_tuning(emf_solver *s, int kind, int tyg, int zc, int order)
     s->kind = kind;
     s->tyg = tyg;
     s->zc = zc;
+    s->zc_auto = false;
     s->order = order;
     return EMF_OK;
 }

@@ -36,6 +36,7 @@ struct Geo {
     int bc[3];           // '0', 'E', 'H' per axis x, y, z
     int zc;              // z planes per work-group
     int order;           // work-group order of the two passes (see pass_tile)
+    int strip = 0;       // order 3: rows of a strip, 0 for none
 };
 
 // CPML coefficient tables of one pass (H uses the *_H_* set, E the *_E_*).

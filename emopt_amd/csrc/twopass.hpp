@@ -29,18 +29,43 @@ constexpr int PX = 64;
 // z fastest, then x, then y.  order 2: as 1, after regrouping the linear id
 // by XCD (the dispatcher deals consecutive work-groups to the 8 XCDs in turn),
 // so that z-neighbouring tiles, which share a halo plane, run on one XCD and
-// share its L2.  order 3: as 0, but the E pass (rev) walks the tiles
-// backwards, so that each pass starts where the previous one ended and
-// first reads what that pass wrote last, while it is still in the Infinity
-// Cache.  The mapping is a bijection for any work-group count.
+// share its L2.  order 3: the E pass (rev) walks the tiles backwards, so that
+// each pass starts where the previous one ended and first reads what that
+// pass wrote last; the tiles are dealt in one of two ways:
+//
+// g.strip == 0: as 0, for data past the Infinity Cache.  The chip sweeps
+// the grid as one front, which is what the memory channels take best
+// (400x200x120: 299 us a step, 328 with strips), and what the H pass left in
+// the Infinity Cache is read again by the E pass.
+//
+// g.strip > 0: for data within it.  The tiles in the order strip of rows,
+// plane, row, x are cut into one contiguous range per XCD, the same one in both
+// passes: the planes and rows that tiles share are then in the L2 of the
+// XCD that needs them again (the strip's few planes fit there), instead
+// of being read by up to four XCDs.  us a step, 0 -> strips: 180x60x80 37.4
+// -> 31.5, 173x101x67 with complex eps 56.5 -> 43.4, 200x100x100 74 -> 64,
+// 360x60x120 85 -> 72, 400x100x100 116 -> 100; strips of 16 rows or of 64 and
+// more are 2 to 6 % slower than those of about 40.
+//
+// The mapping is a bijection for any work-group count.
 __device__ __forceinline__ void pass_tile(const Geo &g, int ty, int &k, int &j, int &z0, int &z1,
                                           bool rev = false)
 {
     const unsigned nbx = gridDim.x, nby = gridDim.y, nbz = gridDim.z;
     unsigned l = blockIdx.x + nbx * (blockIdx.y + nby * blockIdx.z);
-    if (rev && g.order == 3) l = nbx * nby * nbz - 1 - l;
+    const bool strips = g.order == 3 && g.strip > 0;
+    if (rev && g.order == 3 && !strips) l = nbx * nby * nbz - 1 - l;
     unsigned bx, by, bz;
-    if (g.order == 0 || g.order == 3) {
+    if (strips) {
+        const unsigned nb = nbx * nby * nbz, q = nb / 8, r = nb % 8;
+        const unsigned xcd = l % 8, c = xcd < r ? q + 1 : q, slot = l / 8;
+        l = xcd * q + min(xcd, r) + (rev ? c - 1 - slot : slot);
+        const unsigned Y = max(1u, (unsigned)(g.strip / ty)), sb = l / (Y * nbz * nbx);
+        const unsigned yn = min(Y, nby - sb * Y);
+        l -= sb * Y * nbz * nbx;
+        bx = l % nbx; l /= nbx;
+        by = sb * Y + l % yn; bz = l / yn;
+    } else if (g.order == 0 || g.order == 3) {
         bx = l % nbx; by = (l / nbx) % nby; bz = l / (nbx * nby);
     } else {
         if (g.order == 2) {
@@ -349,7 +374,7 @@ __device__ __forceinline__ void e_column(const FusedArgs &A, const Geo &g, const
     }
 }
 
-// ZU: see e_column (the launch picks the smallest ZU of 2, 4, 8 that holds
+// ZU: see e_column (the launch picks the smallest ZU of 1, 2, 4, 8 that holds
 // zc).  BIG: as for k_pass_h.
 template <int CM, int TY, int OCC = 4, int ZU = 0, bool NT = false, bool BIG = false>
 __global__ __launch_bounds__(PX * TY, OCC) void k_pass_e(FusedArgs A, Geo g, PassSrc se,
