@@ -1062,26 +1062,40 @@ int phasor3(emf_solver *s, int slot, double t0, double t1, double t2)
 // How a grid is split into boxes: GX x GY x GZ of them, NZ planes per thread.
 struct ResPlan {
     int NZ = 0, GX = 0, GY = 0, GZ = 0, BX = 0, BY = 0, threads = 0;
+    bool deep = false;
     size_t lds = 0;
     int boxes() const { return GX * GY * GZ; }
 };
 
 constexpr size_t kResLds = 160 * 1024;
 
-int res_max_planes(const emf_solver *s) { return s->ceps || !s->mu_uniform ? 3 : 5; }
+// Whether some box of the split meets both slabs of an axis, of different widths.
+bool res_two_widths(int N, int G, int lo, int hi)
+{
+    if (lo == hi || lo == 0 || hi == 0) return false;
+    for (int b = 0; b < G; ++b) {
+        const int a = (int)((long long)b * N / G), e = (int)((long long)(b + 1) * N / G);
+        if (a < lo && e > N - hi) return true;
+    }
+    return false;
+}
 
-// Fills the plan for boxes of this split; false where the kernel cannot take it.
+// Fills the plan for boxes of this split; false where no kernel takes it.
 bool res_split(const emf_solver *s, int GX, int GY, int GZ, ResPlan &r)
 {
     r.GX = GX; r.GY = GY; r.GZ = GZ;
     r.BX = (s->Nx + GX - 1) / GX; r.BY = (s->Ny + GY - 1) / GY; r.NZ = (s->Nz + GZ - 1) / GZ;
-    if (r.NZ > res_max_planes(s) || r.BX > RES_W || r.BY > RES_W || r.BX * r.BY > RES_T ||
-        (r.BX + 1) * (r.BY + 1) > RES_PL)
+    r.deep = r.NZ > res_planes(s->ceps, !s->mu_uniform);
+    if (r.NZ > res_planes_deep(!s->mu_uniform) || r.BX > RES_W ||
+        r.BY > RES_W || r.BX * r.BY > RES_T || (r.BX + 1) * (r.BY + 1) > RES_PL)
         return false;
-    // a thread per column, and RES_ITEMS halo slots of the x and y faces per thread
-    const int items = 2 * r.NZ * (r.BX + r.BY);
-    r.threads = (std::max(r.BX * r.BY, (items + RES_ITEMS - 1) / RES_ITEMS) + 63) / 64 * 64;
-    r.lds = res_lds(r.NZ, r.BX, r.BY);
+    if (r.deep && (res_two_widths(s->Nx, GX, s->w[0], s->w[1]) ||
+                   res_two_widths(s->Ny, GY, s->w[2], s->w[3])))
+        return false;
+    // a thread per column, and res_items halo slots of the x and y faces per thread
+    const int items = 2 * r.NZ * (r.BX + r.BY), it = res_items(r.deep);
+    r.threads = (std::max(r.BX * r.BY, (items + it - 1) / it) + 63) / 64 * 64;
+    r.lds = res_lds(r.NZ, r.deep, r.BX, r.BY);
     return r.threads <= RES_T && r.lds <= kResLds;
 }
 
@@ -1098,12 +1112,12 @@ bool resident_plan(const emf_solver *s, int ncu, ResPlan &best)
     if (s->res_off || s->kind != 1 || s->wide || s->Nx < 2 || s->Ny < 2 || s->Nz < 2) return false;
     double bt = 1e30;
     for (int GZ = 1; GZ <= std::min(ncu, s->Nz); ++GZ) {
-        if ((s->Nz + GZ - 1) / GZ > res_max_planes(s)) continue;
+        if ((s->Nz + GZ - 1) / GZ > res_planes_deep(!s->mu_uniform)) continue;
         for (int GY = 1; GY <= std::min(ncu / GZ, s->Ny); ++GY)
             for (int GX = 1; GX <= std::min(ncu / (GZ * GY), s->Nx); ++GX) {
                 ResPlan r;
                 if (!res_split(s, GX, GY, GZ, r)) continue;
-                const double t = 0.15 * r.NZ * (r.threads / 64) + 0.02 * r.NZ * r.BY;
+                const double t = (r.deep ? 2.0 : 1.0) * (0.15 * r.NZ * (r.threads / 64) + 0.02 * r.NZ * r.BY);
                 if (t < bt) { bt = t; best = r; }
             }
     }
@@ -1194,9 +1208,16 @@ int res_launch_nz(emf_solver *s, const ResPlan &r, const ResArgs &R, const Fused
     case 2: return res_launch_t<2, CE, MU>(s, r, R, A, g, done);
     case 3: return res_launch_t<3, CE, MU>(s, r, R, A, g, done);
     }
-    if constexpr (!CE && !MU) {
-        if (r.NZ == 4) return res_launch_t<4, CE, MU>(s, r, R, A, g, done);
-        return res_launch_t<5, CE, MU>(s, r, R, A, g, done);
+    if constexpr (!MU) {
+        switch (r.NZ) {
+        case 4: return res_launch_t<4, CE, MU>(s, r, R, A, g, done);
+        case 5: return res_launch_t<5, CE, MU>(s, r, R, A, g, done);
+        case 6: return res_launch_t<6, CE, MU>(s, r, R, A, g, done);
+        case 7: return res_launch_t<7, CE, MU>(s, r, R, A, g, done);
+        case 8: return res_launch_t<8, CE, MU>(s, r, R, A, g, done);
+        case 9: return res_launch_t<9, CE, MU>(s, r, R, A, g, done);
+        case 10: return res_launch_t<10, CE, MU>(s, r, R, A, g, done);
+        }
     }
     EMF_FAIL(EMF_ERR_ARG, "no resident kernel for %d planes", r.NZ);
 }

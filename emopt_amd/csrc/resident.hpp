@@ -1,8 +1,9 @@
 // Resident solve steps: many time steps per launch with the whole state of the
 // grid held in registers.
 //
-// A grid of up to about a million cells fits the vector registers of the chip
-// (512 KB per CU).  Each work-group owns one box of cells, one (x, y) column of
+// A grid of up to 655 thousand cells fits the vector registers of the chip
+// (512 KB per CU) with its CPML psi and coefficients, one of up to 1.3 million
+// without them.  Each work-group owns one box of cells, one (x, y) column of
 // up to NZ planes per thread, loads E, H and the coefficients once, and takes
 // `nsteps` steps; only the box faces travel between work-groups, through halo
 // slots in device memory, and only neighbours wait for each other.  x and y
@@ -33,7 +34,6 @@ namespace emf {
 
 constexpr int RES_T = 512;            // threads of the largest box
 constexpr int RES_STEPS = 64;         // steps per launch (their factors travel as arguments)
-constexpr int RES_ITEMS = 1;          // x and y halo slots polled per thread
 constexpr int RES_SPIN = 1 << 21;     // polls before a launch counts as stalled (seconds; ResArgs::spin)
 constexpr int RES_PL = 592;           // doubles of one LDS plane: (BX + 1) (BY + 1) at most
 constexpr int RES_W = 64;             // largest box width in x and in y
@@ -52,14 +52,29 @@ struct ResArgs {
     double fac[RES_STEPS][6];         // per step: sin t, cos t, env(t) of the H and E halves
 };
 
-// E and H share one LDS buffer (two more barriers per step), and the E
-// coefficients live in LDS, where the registers are full
-constexpr bool res_tight(int nz) { return nz > 4; }
+// Planes per thread with the whole state in registers; boxes with more planes
+// are deep: only the fields stay in registers, psi and the E coefficients
+// (which a step reads once) are read from memory, where each box's part
+// stays in the L2 of its XCD or in the Infinity Cache, one plane ahead of
+// their use.  us a step, two passes -> deep: 118x78x66 26.2 -> 16.3, 180x60x80
+// 31.9 -> 20.3, 152x100x68 37.3 -> 25.3, 173x101x67 with complex eps 42.8 ->
+// 30.2; of these about 6 us are psi's loads and stores and 1 to 6 the
+// coefficients.  8 planes and more spill some registers (20 to 60).
+constexpr int res_planes(bool ceps, bool mu) { return ceps || mu ? 3 : 5; }
+// Deepest boxes.  Complex eps reads 24 B a cell more; non-uniform mu has no deep kernel.
+constexpr int res_planes_deep(bool mu) { return mu ? 3 : 10; }
+// x and y halo slots polled per thread
+constexpr int res_items(bool deep) { return deep ? 2 : 1; }
 
-constexpr size_t res_lds(int nz, int bx, int by)
+// E and H share one LDS buffer (two more barriers per step) where the planes
+// of both do not fit, and the E coefficients live in LDS, where the registers are full
+constexpr bool res_share(int nz, bool deep) { return deep || nz > 4; }
+constexpr bool res_tight(int nz, bool deep) { return !deep && nz > 4; }
+
+constexpr size_t res_lds(int nz, bool deep, int bx, int by)
 {
-    return 8 * ((size_t)(res_tight(nz) ? 3 : 6) * nz * RES_PL + (res_tight(nz) ? 3 * nz * RES_T : 0) +
-                6 * (size_t)(bx + by + nz) + 6 * RES_STEPS);
+    return 8 * ((size_t)(res_share(nz, deep) ? 3 : 6) * nz * RES_PL +
+                (res_tight(nz, deep) ? 3 * nz * RES_T : 0) + 6 * (size_t)(bx + by + nz) + 6 * RES_STEPS);
 }
 
 // halo slots of one box, field and parity: x face [component][plane][RES_W],
@@ -90,6 +105,7 @@ __device__ __forceinline__ void slot_put(unsigned long long *base, unsigned off,
 // step loop is computed there: hoisted out of the loop, the addresses of every
 // plane would take the registers that hold the state.
 __device__ __forceinline__ void fresh(unsigned &v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void fresh_uniform(unsigned &v) { asm volatile("" : "+s"(v)); }
 
 // CPML of one derivative: d becomes ki d + psi with psi <- c d + b psi
 __device__ __forceinline__ void res_stretch(double &d, double &psi, double c, double b, double ki)
@@ -98,13 +114,25 @@ __device__ __forceinline__ void res_stretch(double &d, double &psi, double c, do
     d = ki * d + psi;
 }
 
+// the same with psi as it is in memory: c carries the spacing factor r of the axis, ri = 1 / r
+__device__ __forceinline__ void res_stretch(double &d, double &psi, double c, double b, double ki,
+                                            double ri)
+{
+    psi = c * d + b * psi;
+    d = fma(ri, psi, ki * d);
+}
+
 template <int NZ, bool CEPS, bool MU>
 __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, Geo g,
                                                        const int *__restrict__ done)
 {
     extern __shared__ double lds[];
     if (done && *done) return;
-    constexpr bool TIGHT = res_tight(NZ);
+    constexpr bool DEEP = NZ > res_planes(CEPS, MU);
+    constexpr bool TIGHT = res_tight(NZ, DEEP), SHARE = res_share(NZ, DEEP);
+    constexpr int ITEMS = res_items(DEEP);
+    constexpr int NP = DEEP ? 1 : NZ;     // planes of the arrays that deep boxes keep in memory
+    static_assert(!(DEEP && MU), "no deep kernel with a mu array");
     constexpr int comp = NZ * RES_PL;
     const int Nx = g.Nx, Ny = g.Ny, Nz = g.Nz;
     const int GX = R.GX, GY = R.GY, GZ = R.GZ, nb = GX * GY * GZ;
@@ -125,7 +153,7 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
     // LDS: E (halo column at x = xw, row at y = yw), H (halo column and row at
     // -1, stored shifted by one), E coefficients, CPML coefficients (H c, b,
     // 1/kappa, E c, b, 1/kappa) by x, y and plane, step factors
-    double *const eb = lds, *const hb = TIGHT ? eb : eb + 3 * comp;
+    double *const eb = lds, *const hb = SHARE ? eb : eb + 3 * comp;
     double *const bb = hb + 3 * comp;
     double *const xc = bb + (TIGHT ? 3 * NZ * RES_T : 0);
     double *const yc = xc + 6 * R.BX, *const zc = yc + 6 * R.BY, *const fac = zc + 6 * NZ;
@@ -144,10 +172,11 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
             if (a == 2 && u >= zw) s.in = false;
             double *const c = (a == 0 ? xc : (a == 1 ? yc : zc)) + 6 * u;
             const unsigned t = L.tbo[a] + (s.in ? (unsigned)s.par * 8u : 0u), n = L.tbl[a];
-            c[0] = s.in ? ldc(A.tab, t + 2 * n) : 0.0;
+            const double ra = !DEEP ? 1.0 : (a == 0 ? g.rx : (a == 1 ? g.ry : g.rz));
+            c[0] = s.in ? ra * ldc(A.tab, t + 2 * n) : 0.0;
             c[1] = s.in ? ldc(A.tab, t + n) : 0.0;
             c[2] = s.in ? 1.0 / ldc(A.tab, t) : 1.0;
-            c[3] = s.in ? ldc(A.tab, t + 5 * n) : 0.0;
+            c[3] = s.in ? ra * ldc(A.tab, t + 5 * n) : 0.0;
             c[4] = s.in ? ldc(A.tab, t + 4 * n) : 0.0;
             c[5] = s.in ? 1.0 / ldc(A.tab, t + 3 * n) : 1.0;
         }
@@ -159,17 +188,17 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
     // state.  The E coefficients carry one of the curl's two spacing factors
     // (the other enters as a ratio, 1 on a cubic grid), the H ones both.
     double ex[NZ], ey[NZ], ez[NZ], hx[NZ], hy[NZ], hz[NZ];
-    double b0[TIGHT ? 1 : NZ], b1[TIGHT ? 1 : NZ], b2[TIGHT ? 1 : NZ];
-    double a0[CEPS ? NZ : 1], a1[CEPS ? NZ : 1], a2[CEPS ? NZ : 1];
+    double b0[TIGHT ? 1 : NP], b1[TIGHT ? 1 : NP], b2[TIGHT ? 1 : NP];
+    double a0[CEPS ? NP : 1], a1[CEPS ? NP : 1], a2[CEPS ? NP : 1];
     double m0[MU ? NZ : 1], m1[MU ? NZ : 1], m2[MU ? NZ : 1];
     // psi of d/dx of the y and z components, d/dy of x and z, d/dz of x and y,
     // in units of the undivided differences
-    double px0[NZ], px1[NZ], py0[NZ], py1[NZ], pz0[NZ], pz1[NZ];
-    double qx0[NZ], qx1[NZ], qy0[NZ], qy1[NZ], qz0[NZ], qz1[NZ];
+    double px0[NP], px1[NP], py0[NP], py1[NP], pz0[NP], pz1[NP];
+    double qx0[NP], qx1[NP], qy0[NP], qy1[NP], qz0[NP], qz1[NP];
     // f(offset, H psi, E psi, axis) of every psi of the column
     auto each_psi = [&](auto &&f) {
 #pragma unroll
-        for (int q = 0; q < NZ; ++q) {
+        for (int q = 0; q < NP; ++q) {
             if (q >= zw) break;
             __builtin_amdgcn_sched_barrier(0);
             const Slab sx = slab_x(g, z0 + q, j, k), sy = slab_y(g, z0 + q, j, k),
@@ -194,8 +223,16 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
         const unsigned c = o + (unsigned)q * oz;
         const bool v = on && q < zw;
         ex[q] = ey[q] = ez[q] = hx[q] = hy[q] = hz[q] = 0;
-        px0[q] = px1[q] = py0[q] = py1[q] = pz0[q] = pz1[q] = 0;
-        qx0[q] = qx1[q] = qy0[q] = qy1[q] = qz0[q] = qz1[q] = 0;
+        if (DEEP) {
+            if (v) {
+                ex[q] = ldo(A.Eo, c); ey[q] = ldo(A.Eo, c + cs); ez[q] = ldo(A.Eo, c + 2 * cs);
+                hx[q] = ldo(A.Ho, c); hy[q] = ldo(A.Ho, c + cs); hz[q] = ldo(A.Ho, c + 2 * cs);
+            }
+            continue;
+        }
+        const int u = DEEP ? 0 : q;
+        px0[u] = px1[u] = py0[u] = py1[u] = pz0[u] = pz1[u] = 0;
+        qx0[u] = qx1[u] = qy0[u] = qy1[u] = qz0[u] = qz1[u] = 0;
         double u0 = 0, u1 = 0, u2 = 0;
         if (v) {
             ex[q] = ldo(A.Eo, c); ey[q] = ldo(A.Eo, c + cs); ez[q] = ldo(A.Eo, c + 2 * cs);
@@ -207,18 +244,18 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
             bb[(3 * q + 1) * RES_T + p] = u1;
             bb[(3 * q + 2) * RES_T + p] = u2;
         } else {
-            b0[TIGHT ? 0 : q] = u0; b1[TIGHT ? 0 : q] = u1; b2[TIGHT ? 0 : q] = u2;
+            b0[TIGHT ? 0 : u] = u0; b1[TIGHT ? 0 : u] = u1; b2[TIGHT ? 0 : u] = u2;
         }
         if (CEPS) {
-            a0[q] = v ? ldo(A.aE, c) : 0; a1[q] = v ? ldo(A.aE, c + cs) : 0;
-            a2[q] = v ? ldo(A.aE, c + 2 * cs) : 0;
+            a0[u] = v ? ldo(A.aE, c) : 0; a1[u] = v ? ldo(A.aE, c + cs) : 0;
+            a2[u] = v ? ldo(A.aE, c + 2 * cs) : 0;
         }
         if (MU) {
             m0[q] = v ? ldo(A.mH, c) : 0; m1[q] = v ? ldo(A.mH, c + cs) : 0;
             m2[q] = v ? ldo(A.mH, c + 2 * cs) : 0;
         }
     }
-    if (hasx || hasy || hasz)
+    if (!DEEP && (hasx || hasy || hasz))
         each_psi([&](unsigned off, double &ph, double &pe, int a) {
             const double ri = a == 0 ? 1.0 / rx : (a == 1 ? 1.0 / ry : 1.0 / rz);
             ph = ldo(A.pho, off) * ri;
@@ -232,11 +269,11 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
     constexpr unsigned QB = 8u * RES_W;           // bytes to the next plane of a face
     const unsigned fb = (unsigned)nb * SB;        // to the next field
     const unsigned own = (unsigned)bl * SB;
-    unsigned slot[RES_ITEMS], pos[RES_ITEMS];   // byte offset of the slot; LDS byte of the E halo
-    int dpos[RES_ITEMS];                        // from the E to the H place
-    bool oke[RES_ITEMS], okh[RES_ITEMS];        // there is a neighbour on that side
+    unsigned slot[ITEMS], pos[ITEMS];   // byte offset of the slot; LDS byte of the E halo
+    int dpos[ITEMS];                        // from the E to the H place
+    bool oke[ITEMS], okh[ITEMS];        // there is a neighbour on that side
 #pragma unroll
-    for (int it = 0; it < RES_ITEMS; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int t = p + it * nt, nxi = 2 * NZ * yw;
         slot[it] = own;
         pos[it] = 0;
@@ -264,19 +301,19 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
 
     // wait for the halo of the field and parity at byte offset f: the x and y
     // slots xy, returned in v, and the two z neighbours of the column (zon)
-    auto recv = [&](unsigned f, const bool (&xy)[RES_ITEMS], bool zon, double (&vd)[RES_ITEMS],
+    auto recv = [&](unsigned f, const bool (&xy)[ITEMS], bool zon, double (&vd)[ITEMS],
                     double &z0v, double &z1v) {
-        unsigned long long v[RES_ITEMS] = {}, a = 0, b = 0;
+        unsigned long long v[ITEMS] = {}, a = 0, b = 0;
         const unsigned sz = f + zslot;
         for (int spin = 1;; ++spin) {
 #pragma unroll
-            for (int it = 0; it < RES_ITEMS; ++it)
+            for (int it = 0; it < ITEMS; ++it)
                 if (xy[it]) v[it] = slot_load(R.halo, f + slot[it]);
             if (zon) { a = slot_load(R.halo, sz); b = slot_load(R.halo, sz + ZB); }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             bool miss = a == RES_EMPTY || b == RES_EMPTY;
 #pragma unroll
-            for (int it = 0; it < RES_ITEMS; ++it) miss |= v[it] == RES_EMPTY;
+            for (int it = 0; it < ITEMS; ++it) miss |= v[it] == RES_EMPTY;
             if (!miss || dead) break;
             if (spin >= R.spin) {
                 __hip_atomic_store(&R.conv->stalled, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -287,7 +324,7 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
             }
         }
 #pragma unroll
-        for (int it = 0; it < RES_ITEMS; ++it) {
+        for (int it = 0; it < ITEMS; ++it) {
             if (xy[it]) slot_store(R.halo, f + slot[it], RES_EMPTY);
             vd[it] = __longlong_as_double(v[it]);
         }
@@ -411,8 +448,9 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
     // curl factors: H coefficients times the spacing factors, and the ratios of the E update
     const double sx = MU ? rx : A.m_s * rx, sy = MU ? ry : A.m_s * ry, sz = MU ? rz : A.m_s * rz;
     const double ryz = ry / rz, rzx = rz / rx, rxy = rx / ry;
-    auto coef = [&](const double (&f)[TIGHT ? 1 : NZ], int c, int q) {
-        return TIGHT ? bb[(3 * q + c) * RES_T + p] : f[TIGHT ? 0 : q];
+    auto coef = [&](const double (&f)[TIGHT ? 1 : NP], int c, int q) {
+        if (DEEP) return ldo(A.bE, o + (unsigned)q * oz + (unsigned)c * cs) * (c == 0 ? rz : (c == 1 ? rx : ry));
+        return TIGHT ? bb[(3 * q + c) * RES_T + p] : f[TIGHT || DEEP ? 0 : q];
     };
     // plane q + 1 of an E component: the column's own, past its top the neighbour's
     auto above = [&](const double (&f)[NZ], int q, double top) {
@@ -420,6 +458,90 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
         const double v = f[q + 1 < NZ ? q + 1 : q];
         return q + 2 < NZ || full ? v : top;
     };
+    // Deep boxes: psi and coefficients of this thread's cells in memory, through
+    // buffer accesses, whose range check makes the code straight: a cell that
+    // has no such value has the offset NONE, which loads 0 and stores nothing.
+    // A box that meets both faces of an axis has slabs of one width there.
+    constexpr unsigned NONE = 0x80000000u;   // past every array, also with what is added to it
+    unsigned ox_ = NONE, oy_ = NONE, oz_ = NONE;
+    unsigned dxs = 0, dxc = 0, dys = 0, dyc = 0;       // to the next plane and the second array
+    unsigned zin = 0, zlo = 0, za0 = 0, za1 = 0, zb0 = 0, zb1 = 0;   // planes in a z slab, in the min one; plane z0 in each
+    if (DEEP) {
+        const Slab a = slab_x(g, z0, j, k), b = slab_y(g, z0, j, k);
+        if (on && a.in) ox_ = psof(L, 0, a.lo, 0) + a.io;
+        if (on && b.in) oy_ = psof(L, 1, b.lo, 0) + b.io;
+        if (on) oz_ = ((unsigned)j * (unsigned)Nx + (unsigned)k) * 8u;
+        const unsigned wx = (unsigned)(x0 < g.w[0] ? g.w[0] : g.w[1]), wy = (unsigned)(y0 < g.w[2] ? g.w[2] : g.w[3]);
+        dxs = (unsigned)Ny * wx * 8u; dxc = (unsigned)Nz * dxs;
+        dys = (unsigned)Nx * wy * 8u; dyc = (unsigned)Nz * dys;
+        for (int q = 0; q < zw; ++q) {
+            const Slab z = slab_z(g, z0 + q, 0, 0);
+            zin |= z.in ? 1u << q : 0u;
+            zlo |= z.lo ? 1u << q : 0u;
+        }
+        za0 = psof(L, 2, true, 0) + (unsigned)z0 * oz; za1 = psof(L, 2, true, 1) + (unsigned)z0 * oz;
+        zb0 = psof(L, 2, false, 0) + (unsigned)(z0 - Nz + g.w[5]) * oz;
+        zb1 = psof(L, 2, false, 1) + (unsigned)(z0 - Nz + g.w[5]) * oz;
+    }
+    const unsigned pbytes = 2u * 8u * (unsigned)((g.w[0] + g.w[1]) * Nz * Ny + (g.w[2] + g.w[3]) * Nz * Nx +
+                                                 (g.w[4] + g.w[5]) * Ny * Nx);
+    typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u2;
+    auto buf_get = [](__amdgpu_buffer_rsrc_t r, unsigned v, unsigned so) {
+        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v, (int)so, 0));
+    };
+    auto buf_put = [](__amdgpu_buffer_rsrc_t r, unsigned v, unsigned so, double d) {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, d), r, (int)v, (int)so, 0);
+    };
+    auto rsrc = [](const double *p, unsigned bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, (int)bytes, 0x00020000);
+    };
+    unsigned ozs = oz, css = cs;
+    auto fresh_deep = [&] {
+        fresh(ox_); fresh(oy_); fresh(oz_);
+        fresh_uniform(dxs); fresh_uniform(dxc); fresh_uniform(dys); fresh_uniform(dyc);
+        fresh_uniform(zin); fresh_uniform(zlo);
+        fresh_uniform(za0); fresh_uniform(za1); fresh_uniform(zb0); fresh_uniform(zb1);
+        fresh_uniform(ozs); fresh_uniform(css);
+    };
+    // plane q's psi from, or to, the arrays of one field
+    auto psi_off = [&](int q, unsigned &vx, unsigned &vy, unsigned &vz, unsigned &z0o, unsigned &z1o) {
+        const unsigned spare = q < zw ? 0u : NONE;
+        vx = ox_ | spare;
+        vy = oy_ | spare;
+        vz = oz_ | ((zin >> q) & 1u ? 0u : NONE);
+        const bool lo = (zlo >> q) & 1u;
+        z0o = (lo ? za0 : zb0) + (unsigned)q * ozs;
+        z1o = (lo ? za1 : zb1) + (unsigned)q * ozs;
+    };
+    auto psi_get = [&](const double *f, int q, double (&v)[6]) {
+        unsigned vx, vy, vz, za, zb;
+        psi_off(q, vx, vy, vz, za, zb);
+        const auto r = rsrc(f, pbytes);
+        v[0] = buf_get(r, vx, (unsigned)q * dxs); v[1] = buf_get(r, vx, (unsigned)q * dxs + dxc);
+        v[2] = buf_get(r, vy, (unsigned)q * dys); v[3] = buf_get(r, vy, (unsigned)q * dys + dyc);
+        v[4] = buf_get(r, vz, za); v[5] = buf_get(r, vz, zb);
+    };
+    auto psi_put = [&](double *f, int q, const double (&v)[6]) {
+        unsigned vx, vy, vz, za, zb;
+        psi_off(q, vx, vy, vz, za, zb);
+        const auto r = rsrc(f, pbytes);
+        buf_put(r, vx, (unsigned)q * dxs, v[0]); buf_put(r, vx, (unsigned)q * dxs + dxc, v[1]);
+        buf_put(r, vy, (unsigned)q * dys, v[2]); buf_put(r, vy, (unsigned)q * dys + dyc, v[3]);
+        buf_put(r, vz, za, v[4]); buf_put(r, vz, zb, v[5]);
+    };
+    // plane q's E coefficients: b and, with complex eps, a (0 where there is no cell)
+    unsigned ob = on ? o : NONE;
+    auto coef_get = [&](int q, double (&v)[CEPS ? 6 : 3]) {
+        const unsigned c = ob | (q < zw ? 0u : NONE), so = (unsigned)q * ozs;
+        const auto r = rsrc(A.bE, 3u * css);
+        v[0] = buf_get(r, c, so); v[1] = buf_get(r, c, so + css); v[2] = buf_get(r, c, so + 2 * css);
+        if (CEPS) {
+            const auto ra = rsrc(A.aE, 3u * css);
+            v[CEPS ? 3 : 0] = buf_get(ra, c, so); v[CEPS ? 4 : 0] = buf_get(ra, c, so + css);
+            v[CEPS ? 5 : 0] = buf_get(ra, c, so + 2 * css);
+        }
+    };
+    const double rix = 1.0 / rx, riy = 1.0 / ry, riz = 1.0 / rz;
     // Every box runs the CPML arithmetic (with psi = 0 and c = b = 0 outside
     // the slabs): a box waits for its neighbours each half step, so the boxes in
     // the corners, which need it on all axes, set the pace, and a straight line
@@ -429,13 +551,17 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
         put_e(fe);
         for (int s = 0; s < R.nsteps; ++s) {
             double zx, zy;
+            double pn[6] = {};        // deep: the next plane's psi
+            double cn[CEPS ? 6 : 3] = {};
             // ------------------------------------------------------ H half
+            if (DEEP) fresh_deep();
             fresh(zslot); fresh(le); fresh(lh); fresh(yx); fresh(yy);
             {
-                double v[RES_ITEMS];
+                double v[ITEMS];
+                if (DEEP) psi_get(A.pho, 0, pn);
                 recv(fe, oke, on && bz + 1 < GZ, v, zx, zy);
 #pragma unroll
-                for (int it = 0; it < RES_ITEMS; ++it)
+                for (int it = 0; it < ITEMS; ++it)
                     if (oke[it]) E(0, 0, pos[it]) = v[it];
             }
             __syncthreads();
@@ -450,12 +576,27 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
                     double dzy_ = above(ey, q, zy) - ey[q], dyz_ = E(2, q, lr) - ez[q];
                     double dxz_ = E(2, q, le + 8u) - ez[q], dzx_ = above(ex, q, zx) - ex[q];
                     double dyx_ = E(0, q, lr) - ex[q], dxy_ = E(1, q, le + 8u) - ey[q];
-                    res_stretch(dzy_, pz1[q], cz, bz_, kz);
-                    res_stretch(dzx_, pz0[q], cz, bz_, kz);
-                    res_stretch(dyz_, py1[q], cy, by_, ky);
-                    res_stretch(dyx_, py0[q], cy, by_, ky);
-                    res_stretch(dxz_, px1[q], cx, bx_, kx);
-                    res_stretch(dxy_, px0[q], cx, bx_, kx);
+                    if (DEEP) {
+                        double pc[6];
+#pragma unroll
+                        for (int n = 0; n < 6; ++n) pc[n] = pn[n];
+                        if (q + 1 < NZ) psi_get(A.pho, q + 1, pn);
+                        res_stretch(dzy_, pc[5], cz, bz_, kz, riz);
+                        res_stretch(dzx_, pc[4], cz, bz_, kz, riz);
+                        res_stretch(dyz_, pc[3], cy, by_, ky, riy);
+                        res_stretch(dyx_, pc[2], cy, by_, ky, riy);
+                        res_stretch(dxz_, pc[1], cx, bx_, kx, rix);
+                        res_stretch(dxy_, pc[0], cx, bx_, kx, rix);
+                        psi_put(A.phn, q, pc);
+                    } else {
+                        const int u = DEEP ? 0 : q;
+                        res_stretch(dzy_, pz1[u], cz, bz_, kz);
+                        res_stretch(dzx_, pz0[u], cz, bz_, kz);
+                        res_stretch(dyz_, py1[u], cy, by_, ky);
+                        res_stretch(dyx_, py0[u], cy, by_, ky);
+                        res_stretch(dxz_, px1[u], cx, bx_, kx);
+                        res_stretch(dxy_, px0[u], cx, bx_, kx);
+                    }
                     if (MU) {
                         hx[q] = fma(m0[MU ? q : 0], sz * dzy_ - sy * dyz_, hx[q]);
                         hy[q] = fma(m1[MU ? q : 0], sx * dxz_ - sz * dzx_, hy[q]);
@@ -474,15 +615,17 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
                             hy[q] += vy * (MU ? m1[MU ? q : 0] : A.m_s);
                             hz[q] += vz * (MU ? m2[MU ? q : 0] : A.m_s);
                         });
-            if (TIGHT) __syncthreads();
+            if (SHARE) __syncthreads();
             put_h(fe + fb);
             // ------------------------------------------------------ E half
+            if (DEEP) { fresh_deep(); fresh(ob); }
             fresh(zslot); fresh(le); fresh(lh); fresh(yx); fresh(yy);
             {
-                double v[RES_ITEMS];
+                double v[ITEMS];
+                if (DEEP) { psi_get(A.pe, 0, pn); coef_get(0, cn); }
                 recv(fe + fb, okh, on && bz > 0, v, zx, zy);
 #pragma unroll
-                for (int it = 0; it < RES_ITEMS; ++it)
+                for (int it = 0; it < ITEMS; ++it)
                     if (okh[it]) H(0, 0, pos[it] + (unsigned)dpos[it]) = v[it];
             }
             if (bz == 0) { const double sg = sign(g.bc[2]); zx = sg * hx[0]; zy = sg * hy[0]; }
@@ -499,18 +642,38 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
                     double dyz_ = hz[q] - H(2, q, lr), dzy_ = hy[q] - (q > 0 ? hy[n] : zy);
                     double dzx_ = hx[q] - (q > 0 ? hx[n] : zx), dxz_ = hz[q] - H(2, q, lx);
                     double dxy_ = hy[q] - H(1, q, lx), dyx_ = hx[q] - H(0, q, lr);
-                    res_stretch(dyz_, qy1[q], cy, by_, ky);
-                    res_stretch(dyx_, qy0[q], cy, by_, ky);
-                    res_stretch(dzy_, qz1[q], cz, bz_, kz);
-                    res_stretch(dzx_, qz0[q], cz, bz_, kz);
-                    res_stretch(dxz_, qx1[q], cx, bx_, kx);
-                    res_stretch(dxy_, qx0[q], cx, bx_, kx);
-                    ex[q] = fma(fma(ryz, dyz_, -dzy_), coef(b0, 0, q),
-                                CEPS ? a0[CEPS ? q : 0] * ex[q] : ex[q]);
-                    ey[q] = fma(fma(rzx, dzx_, -dxz_), coef(b1, 1, q),
-                                CEPS ? a1[CEPS ? q : 0] * ey[q] : ey[q]);
-                    ez[q] = fma(fma(rxy, dxy_, -dyx_), coef(b2, 2, q),
-                                CEPS ? a2[CEPS ? q : 0] * ez[q] : ez[q]);
+                    if (DEEP) {
+                        double pc[6], cc[CEPS ? 6 : 3];
+#pragma unroll
+                        for (int n = 0; n < 6; ++n) pc[n] = pn[n];
+#pragma unroll
+                        for (int n = 0; n < (CEPS ? 6 : 3); ++n) cc[n] = cn[n];
+                        if (q + 1 < NZ) { psi_get(A.pe, q + 1, pn); coef_get(q + 1, cn); }
+                        res_stretch(dyz_, pc[3], cy, by_, ky, riy);
+                        res_stretch(dyx_, pc[2], cy, by_, ky, riy);
+                        res_stretch(dzy_, pc[5], cz, bz_, kz, riz);
+                        res_stretch(dzx_, pc[4], cz, bz_, kz, riz);
+                        res_stretch(dxz_, pc[1], cx, bx_, kx, rix);
+                        res_stretch(dxy_, pc[0], cx, bx_, kx, rix);
+                        psi_put(A.pe, q, pc);
+                        ex[q] = fma(fma(ry, dyz_, -(rz * dzy_)), cc[0],
+                                    CEPS ? cc[CEPS ? 3 : 0] * ex[q] : ex[q]);
+                        ey[q] = fma(fma(rz, dzx_, -(rx * dxz_)), cc[1],
+                                    CEPS ? cc[CEPS ? 4 : 0] * ey[q] : ey[q]);
+                        ez[q] = fma(fma(rx, dxy_, -(ry * dyx_)), cc[2],
+                                    CEPS ? cc[CEPS ? 5 : 0] * ez[q] : ez[q]);
+                    } else {
+                        const int u = DEEP ? 0 : q, w = CEPS ? u : 0;
+                        res_stretch(dyz_, qy1[u], cy, by_, ky);
+                        res_stretch(dyx_, qy0[u], cy, by_, ky);
+                        res_stretch(dzy_, qz1[u], cz, bz_, kz);
+                        res_stretch(dzx_, qz0[u], cz, bz_, kz);
+                        res_stretch(dxz_, qx1[u], cx, bx_, kx);
+                        res_stretch(dxy_, qx0[u], cx, bx_, kx);
+                        ex[q] = fma(fma(ryz, dyz_, -dzy_), coef(b0, 0, q), CEPS ? a0[w] * ex[q] : ex[q]);
+                        ey[q] = fma(fma(rzx, dzx_, -dxz_), coef(b1, 1, q), CEPS ? a1[w] * ey[q] : ey[q]);
+                        ez[q] = fma(fma(rxy, dxy_, -dyx_), coef(b2, 2, q), CEPS ? a2[w] * ez[q] : ez[q]);
+                    }
                 }
             }
             if (anysrc) {
@@ -522,7 +685,7 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
                             ez[q] -= vz * (coef(b2, 2, q) * iy);
                         });
             }
-            if (TIGHT) __syncthreads();
+            if (SHARE) __syncthreads();
             fe = 2u * fb - fe;        // the other parity
             if (s + 1 < R.nsteps) put_e(fe);
         }
@@ -535,7 +698,7 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
             sto(A.Hn, c, hx[q]); sto(A.Hn, c + cs, hy[q]); sto(A.Hn, c + 2 * cs, hz[q]);
         }
     }
-    if (hasx || hasy || hasz)
+    if (!DEEP && (hasx || hasy || hasz))
         each_psi([&](unsigned off, double &ph, double &pe, int a) {
             const double r = a == 0 ? rx : (a == 1 ? ry : rz);
             sto(A.phn, off, ph * r);
