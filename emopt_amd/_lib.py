@@ -95,6 +95,8 @@ _SIGS = {
                                c_double, c_double, c_double, _P], c_int),
     "emf_build_structured": ([_P, _P, c_int, _P, _P, c_int, c_double, c_double, c_double, c_int,
                               c_double, c_double, _P, c_double], c_int),
+    "emf_shape_deps": ([_P, _P, c_int, _P, _P, c_int, c_double, c_double, c_double, c_double, _P, _P,
+                        _P, c_int, _P, c_int, _P, _P, _P, POINTER(c_int)], c_int),
     "emf_copy_bandwidth": ([c_int, c_int64, c_int, _P], c_int),
     "emf_mem_info": ([c_int, POINTER(c_int64), POINTER(c_int64)], c_int),
     "emf_calc_ydAx": ([_P] + [_P] * 6 + [c_int] * 6 + [_P], c_int),

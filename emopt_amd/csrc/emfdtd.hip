@@ -30,6 +30,7 @@
 #include "batch.hpp"
 #include "resident.hpp"
 #include "material.hpp"
+#include "shape.hpp"
 
 using namespace emf;
 
@@ -163,6 +164,8 @@ struct emf_solver {
     double sigma = 3.0, alpha = 0.0, kappa = 1.0, pw = 3.0;
     int bc[3] = { '0', '0', '0' };
     int nconv = 10;
+    unsigned char *shape_ws = nullptr;   // emf_shape_deps' block
+    size_t shape_n = 0;
     int zc = 2;
     bool zc_auto = true;           // zc not chosen by the caller
     int order = 3;                 // two-pass work-group order (pass_tile)
@@ -1584,7 +1587,7 @@ int emf_delete(emf_solver *s)
         dfree(s->samples);
         dfree(s->hist);
         dfree(s->scratch);
-        dfree(s->res_halo);
+        dfree(s->res_halo); dfree(s->shape_ws);
         for (int w = 0; w < emf_solver::kWeightSets; ++w)
             for (int q = 0; q < 6; ++q) dfree(s->wplane[w][q]);
         if (s->done_host) (void)hipHostFree(s->done_host);
@@ -3025,6 +3028,75 @@ int emf_sample_structured(int device, const emf_prim *prims, int nprims, const d
     dfree(dout);
     (void)hipStreamDestroy(st);
     return rc;
+}
+
+int emf_shape_deps(emf_solver *s, const emf_prim *rings, int nrings, const double *vx,
+                   const double *vy, int nverts, double dx, double dy, double bg_re, double bg_im,
+                   const int *seg_off, const int *seg_ring, const int *seg_p, int nseg,
+                   const double *edges, int nedges, const int *box, const double *shifts,
+                   double *out, int *limit)
+{
+    LOCK(s);
+    if (!seg_off || !seg_ring || !seg_p || !edges || !box || !shifts || !out || !limit || nseg < 1 ||
+        nedges < 1)
+        EMF_FAIL(EMF_ERR_ARG, "bad arguments");
+    const MatIn m{ rings, nrings, vx, vy, nverts, dx, dy, 1.0, 0, bg_re, bg_im };
+    CHECK(mat_check(m));
+    for (int q = 0; q < nseg; ++q)
+        if (seg_off[q] < 0 || seg_off[q + 1] < seg_off[q] || seg_p[q] < 0 ||
+            seg_p[q] >= seg_off[q + 1] - seg_off[q])
+            EMF_FAIL(EMF_ERR_ARG, "segment %d: rings out of range", q);
+    const int nlist = seg_off[nseg];
+    for (int q = 0; q < nlist; ++q)
+        if (seg_ring[q] < 0 || seg_ring[q] >= nrings) EMF_FAIL(EMF_ERR_ARG, "ring out of range");
+    ShapeArgs A{};
+    long long total = 0;
+    for (int c = 0; c < 3; ++c) {
+        const int *b = box + 4 * c;
+        if (b[1] < b[0] || b[3] < b[2]) EMF_FAIL(EMF_ERR_ARG, "bad box");
+        A.box[c] = ShapeBox{ total, b[0], b[1] - b[0], b[2], b[3] - b[2], shifts[2 * c], shifts[2 * c + 1] };
+        total += (long long)nseg * (b[1] - b[0]) * (b[3] - b[2]);
+    }
+    *limit = 0;
+    if (total == 0) return EMF_OK;
+    // one block: primitives, vertices, lists, edges, the limit flag, results
+    const size_t o_vx = align_up(nrings * sizeof(MatPrim)), o_vy = align_up(o_vx + nverts * 8);
+    const size_t o_so = align_up(o_vy + nverts * 8), o_sr = align_up(o_so + (nseg + 1) * 4);
+    const size_t o_sp = align_up(o_sr + nlist * 4), o_e = align_up(o_sp + nseg * 4);
+    const size_t o_f = align_up(o_e + nedges * sizeof(ShapeEdge)), o_out = align_up(o_f + 4);
+    std::vector<unsigned char> h(o_out, 0);
+    memcpy(&h[0], rings, nrings * sizeof(MatPrim));
+    if (nverts) { memcpy(&h[o_vx], vx, nverts * 8); memcpy(&h[o_vy], vy, nverts * 8); }
+    memcpy(&h[o_so], seg_off, (nseg + 1) * 4);
+    memcpy(&h[o_sr], seg_ring, nlist * 4);
+    memcpy(&h[o_sp], seg_p, nseg * 4);
+    static_assert(sizeof(ShapeEdge) == 7 * sizeof(double), "edges are seven doubles");
+    memcpy(&h[o_e], edges, nedges * sizeof(ShapeEdge));
+    const size_t bytes = o_out + (size_t)total * sizeof(double2);
+    if (bytes > s->shape_n) {
+        dfree(s->shape_ws);
+        s->shape_n = 0;
+        CHECK(dalloc(&s->shape_ws, bytes));
+        s->shape_n = bytes;
+    }
+    unsigned char *const d = s->shape_ws;
+    A.prims = (const MatPrim *)d;
+    A.vx = (const double *)(d + o_vx); A.vy = (const double *)(d + o_vy);
+    A.seg_off = (const int *)(d + o_so); A.seg_prim = (const int *)(d + o_sr);
+    A.seg_p = (const int *)(d + o_sp); A.edges = (const ShapeEdge *)(d + o_e);
+    A.nseg = nseg; A.nedges = nedges;
+    A.dx = dx; A.dy = dy; A.bg_re = bg_re; A.bg_im = bg_im;
+    HIPCHK(hipMemcpyAsync(d, h.data(), h.size(), hipMemcpyHostToDevice, s->stream));
+    hipLaunchKernelGGL(k_shape_deps, dim3((unsigned)std::min(total, 1LL << 20)), dim3(64), 0, s->stream,
+                       A, total, (double2 *)(d + o_out), (int *)(d + o_f));
+    const hipError_t le = hipGetLastError();
+    if (le == hipSuccess) {
+        (void)hipMemcpyAsync(limit, d + o_f, sizeof(int), hipMemcpyDeviceToHost, s->stream);
+        (void)hipMemcpyAsync(out, d + o_out, (size_t)total * sizeof(double2), hipMemcpyDeviceToHost, s->stream);
+    }
+    HIPCHK(hipStreamSynchronize(s->stream));    // h is done with
+    HIPCHK(le);
+    return EMF_OK;
 }
 
 int emf_build_structured(emf_solver *s, const emf_prim *prims, int nprims, const double *vx,

@@ -40,9 +40,11 @@ Checked cell by cell against central differences of the material sampling
 """
 from __future__ import annotations
 
+from ctypes import byref, c_int
+
 import numpy as np
 
-from .grid import Ellipse, Polygon, Rectangle
+from .grid import Ellipse, Polygon, Rectangle, StructuredMaterial3D
 
 __all__ = ["boundary_deps", "rect_edge_velocity", "polygon_vertex_velocity"]
 
@@ -203,32 +205,75 @@ def boundary_deps(sim, eps, prim, velocity, tol=0.0):
     bg = eps.background
     active_all = [e for e in prims if not isinstance(e[0], Ellipse) or eps._ring(e[0]) is not None]
     bounds = sorted({b for _, z1, z2, _ in active_all for b in (z1, z2)})
+    boxes = []
+    for sx, sy, sz in sim.YEE_SHIFTS[:3]:
+        boxes.append((max(0, int(np.floor(ex0 / dx - sx - 0.5)) - 1),
+                      min(Nx, int(np.ceil(ex1 / dx - sx + 0.5)) + 2),
+                      max(0, int(np.floor(ey0 / dy - sy - 0.5)) - 1),
+                      min(Ny, int(np.ceil(ey1 / dy - sy + 0.5)) + 2)))
+    # the z segments the primitive is in, and their rings in priority order
+    segs = []
+    for za, zb in zip(bounds[:-1], bounds[1:]):
+        if not (entry[1] <= za and entry[2] >= zb):
+            continue
+        active = sorted([e for e in active_all if e[1] <= za and e[2] >= zb],
+                        key=lambda e: (e[0].layer, e[3]))
+        segs.append((za, zb, active))
+    ring_of = {}
+    for _, _, active in segs:
+        for e in active:
+            if id(e) not in ring_of:
+                ring_of[id(e)] = eps._ring(e[0])
+    if getattr(sim, "_h", None) is not None:
+        inplane = _inplane_device(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg)
+    else:
+        inplane = None
+    if inplane is None:
+        inplane = _inplane_host(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg,
+                                (ex0, ex1, ey0, ey1))
     comps, cells, vals = [], [], []
-    for c, (sx, sy, sz) in enumerate(sim.YEE_SHIFTS[:3]):
-        k1 = max(0, int(np.floor(ex0 / dx - sx - 0.5)) - 1)
-        k2 = min(Nx, int(np.ceil(ex1 / dx - sx + 0.5)) + 2)
-        j1 = max(0, int(np.floor(ey0 / dy - sy - 0.5)) - 1)
-        j2 = min(Ny, int(np.ceil(ey1 / dy - sy + 0.5)) + 2)
+    for c, (_, _, sz) in enumerate(sim.YEE_SHIFTS[:3]):
         zc = (np.arange(Nz) + sz) * dz
         zlo, zhi = zc - dz / 2, zc + dz / 2
-        acc = {}
-        for za, zb in zip(bounds[:-1], bounds[1:]):
-            if not (entry[1] <= za and entry[2] >= zb):
-                continue                         # the primitive is not in this segment
+        k1, k2, j1, j2 = boxes[c]
+        cell, val = [], []
+        for (za, zb, _), d2 in zip(segs, inplane[c]):
             fz = np.clip(np.minimum(zhi, zb) - np.maximum(zlo, za), 0, None) / dz
             iz = np.nonzero(fz > 0)[0]
-            if len(iz) == 0:
-                continue
-            active = sorted([e for e in active_all if e[1] <= za and e[2] >= zb],
-                            key=lambda e: (e[0].layer, e[3]))
-            rings, p = [], None
-            for e in active:
-                r = eps._ring(e[0])
-                if r is None:
-                    continue
-                if e[0] is prim:
-                    p = len(rings)
-                rings.append(r)
+            j, k = np.nonzero(d2)
+            cell.append(((iz[None, :] * Ny + (j1 + j)[:, None]) * Nx + (k1 + k)[:, None]).ravel())
+            val.append((fz[iz][None, :] * d2[j, k][:, None]).ravel())
+        if not cell:
+            continue
+        cell, val = np.concatenate(cell), np.concatenate(val)
+        if len(segs) > 1:       # a cell in several segments: their sum, at its first place
+            first, inv = np.unique(cell, return_index=True, return_inverse=True)[1:]
+            total = np.zeros(len(first), dtype=np.complex128)
+            np.add.at(total, inv, val)
+            order = np.argsort(first)
+            cell, val = cell[first[order]], total[order]
+        keep = np.abs(val) > tol
+        if not np.any(keep):
+            continue
+        comps.append(np.full(np.count_nonzero(keep), c, np.int32))
+        cells.append(cell[keep].astype(np.int64))
+        vals.append(val[keep].astype(np.complex128))
+    if not comps:
+        return (np.zeros(0, np.int32), np.zeros(0, np.int64), np.zeros(0, np.complex128))
+    return np.concatenate(comps), np.concatenate(cells), np.concatenate(vals)
+
+
+def _inplane_host(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg, extent):
+    """In-plane derivatives [component][segment][j, k] of the boxes' cells."""
+    ex0, ex1, ey0, ey1 = extent
+    res = []
+    for c, (sx, sy, _) in enumerate(sim.YEE_SHIFTS[:3]):
+        k1, k2, j1, j2 = boxes[c]
+        per = []
+        for _, _, active in segs:
+            rings = [ring_of[id(e)] for e in active]
+            p = next(n for n, e in enumerate(active) if e[0] is prim)
+            d2 = np.zeros((max(0, j2 - j1), max(0, k2 - k1)), dtype=np.complex128)
             for j in range(j1, j2):
                 yc = (j + sy) * dy
                 ya, yb = yc - dy / 2, yc + dy / 2
@@ -239,18 +284,55 @@ def boundary_deps(sim, eps, prim, velocity, tol=0.0):
                     xa, xb = xc - dx / 2, xc + dx / 2
                     if xb < ex0 or xa > ex1:
                         continue
-                    d2 = _inplane_derivative(rings, p, edges, xa, xb, ya, yb, bg)
-                    if d2 == 0.0:
-                        continue
-                    for i in iz:
-                        acc[(i, j, k)] = acc.get((i, j, k), 0.0) + fz[i] * d2
-        keys = [key for key, v in acc.items() if abs(v) > tol]
-        if not keys:
-            continue
-        ijk = np.array(keys, dtype=np.int64)
-        comps.append(np.full(len(keys), c, np.int32))
-        cells.append((ijk[:, 0] * Ny + ijk[:, 1]) * Nx + ijk[:, 2])
-        vals.append(np.array([acc[key] for key in keys], dtype=np.complex128))
-    if not comps:
-        return (np.zeros(0, np.int32), np.zeros(0, np.int64), np.zeros(0, np.complex128))
-    return np.concatenate(comps), np.concatenate(cells), np.concatenate(vals)
+                    d2[j - j1, k - k1] = _inplane_derivative(rings, p, edges, xa, xb, ya, yb, bg)
+            per.append(d2)
+        res.append(per)
+    return res
+
+
+def _inplane_device(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg):
+    """_inplane_host on the solver's GPU (emf_shape_deps), the same doubles;
+    None where a cell counts more primitives than the device holds."""
+    ids, rings = {}, []
+    off, lst, mine = [0], [], []
+    for _, _, active in segs:
+        for n, e in enumerate(active):
+            if id(e) not in ids:
+                ids[id(e)] = len(rings)
+                rings.append(ring_of[id(e)])
+            lst.append(ids[id(e)])
+            if e[0] is prim:
+                mine.append(n)
+        off.append(len(lst))
+    if not segs:
+        return [[], [], []]
+    recs = np.zeros(len(rings), dtype=StructuredMaterial3D.PRIM_DTYPE)
+    nv = 0
+    for r, g in zip(recs, rings):
+        r["kind"], r["v0"], r["nv"] = g.kind, nv, len(g.xs)
+        r["re"], r["im"] = g.value.real, g.value.imag
+        r["bbox"] = g.bbox
+        nv += len(g.xs)
+    vx = np.ascontiguousarray(np.concatenate([g.xs for g in rings]))
+    vy = np.ascontiguousarray(np.concatenate([g.ys for g in rings]))
+    ed = np.array([(P0[0], P0[1], P1[0], P1[1], np.hypot(P1[0] - P0[0], P1[1] - P0[1]),
+                    U0[0] * nrm[0] + U0[1] * nrm[1], U1[0] * nrm[0] + U1[1] * nrm[1])
+                   for P0, P1, U0, U1, nrm in edges], dtype=np.double)
+    box = np.array([(k1, max(k1, k2), j1, max(j1, j2)) for k1, k2, j1, j2 in boxes], dtype=np.int32)
+    sh = np.array([s[:2] for s in sim.YEE_SHIFTS[:3]], dtype=np.double)
+    shape = [(len(segs), b[3] - b[2], b[1] - b[0]) for b in box]
+    out = np.zeros(sum(int(np.prod(s)) for s in shape), dtype=np.complex128)
+    off, lst, mine = (np.array(v, dtype=np.int32) for v in (off, lst, mine))
+    limit = c_int(0)
+    sim._lib.emf_shape_deps(sim._h, recs.ctypes.data, len(recs), vx.ctypes.data, vy.ctypes.data, nv,
+                            dx, dy, bg.real, bg.imag, off.ctypes.data, lst.ctypes.data,
+                            mine.ctypes.data, len(segs), ed.ctypes.data, len(ed), box.ctypes.data,
+                            sh.ctypes.data, out.ctypes.data, byref(limit))
+    if limit.value:
+        return None
+    res, at = [], 0
+    for s in shape:
+        n = int(np.prod(s))
+        res.append(out[at:at + n].reshape(s))
+        at += n
+    return res

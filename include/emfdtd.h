@@ -473,6 +473,21 @@ EMF_API int emf_build_structured(emf_solver *s, const emf_prim *prims, int nprim
                                  double dy, double dz, int supersample, double bg_re,
                                  double bg_im, const double *shifts, double mu_re);
 
+/* In-plane derivatives d(value)/dp of a structured eps under the exact overlap
+ * rule, for a parameter p that moves edges of one primitive.  rings: rectangles
+ * and polygons as emf_prim records (z unused) with their vertices.  Segment s
+ * has the rings seg_ring[seg_off[s] .. seg_off[s + 1]) in priority order, the
+ * moving one being the seg_p[s]-th of them.  edges: per moving edge x0, y0, x1,
+ * y1, length, normal velocity at either end.  box: k1, k2, j1, j2 per eps
+ * component, shifts its in-cell offset (x, y).  out: complex, per component
+ * [segment][j][k].  *limit: nonzero when a cell counts more primitives than the
+ * device holds; out is then incomplete. */
+EMF_API int emf_shape_deps(emf_solver *s, const emf_prim *rings, int nrings, const double *vx,
+                           const double *vy, int nverts, double dx, double dy, double bg_re,
+                           double bg_im, const int *seg_off, const int *seg_ring, const int *seg_p,
+                           int nseg, const double *edges, int nedges, const int *box,
+                           const double *shifts, double *out, int *limit);
+
 typedef struct emf_batch emf_batch;
 
 EMF_API int emf_batch_new(int device, emf_batch **out);
