@@ -1188,6 +1188,28 @@ int res_ready(emf_solver *s, const ResPlan &r)
     return EMF_OK;
 }
 
+// LDS bytes for the source values of a box (res_src_in_lds): what the box with
+// most of them needs, as far as there is room.
+size_t res_src_lds(const emf_solver *s, const ResPlan &r)
+{
+    if (!res_src_in_lds(r.deep, s->ceps)) return 0;
+    size_t most = 0;
+    auto cut = [](int n, int g, int b, int lo, int len) {
+        const int a = std::max(lo, (int)((long long)b * n / g));
+        return (size_t)std::max(0, std::min(lo + len, (int)((long long)(b + 1) * n / g)) - a);
+    };
+    for (int z = 0; z < r.GZ; ++z)
+        for (int y = 0; y < r.GY; ++y)
+            for (int x = 0; x < r.GX; ++x) {
+                size_t need = 0;
+                for (const auto &b : s->srcs)
+                    need += cut(s->Nx, r.GX, x, b.k0, b.K) * cut(s->Ny, r.GY, y, b.j0, b.J) *
+                            cut(s->Nz, r.GZ, z, b.i0, b.I) * 6 * sizeof(double2);
+                most = std::max(most, need);
+            }
+    return std::min(most, kResLds - r.lds) / sizeof(double2) * sizeof(double2);
+}
+
 template <int NZ, bool CE, bool MU>
 int res_launch_t(emf_solver *s, const ResPlan &r, const ResArgs &R, const FusedArgs &A,
                  const Geo &g, const int *done)
@@ -1197,7 +1219,8 @@ int res_launch_t(emf_solver *s, const ResPlan &r, const ResArgs &R, const FusedA
     if (!lds_set.exchange(true))
         HIPCHK(hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)kResLds));
-    hipLaunchKernelGGL(K, dim3(r.boxes()), dim3(r.threads), r.lds, s->stream, R, A, g, done);
+    hipLaunchKernelGGL(K, dim3(r.boxes()), dim3(r.threads), r.lds + (size_t)R.src_cap * sizeof(double2),
+                       s->stream, R, A, g, done);
     HIPCHK(hipGetLastError());
     return EMF_OK;
 }
@@ -1240,6 +1263,7 @@ int res_steps(emf_solver *s, const ResPlan &r, long long n, long long count, con
     R.blk = s->src_desc;
     R.nsrc = (int)s->srcs.size();
     src_union(s, R.ub);
+    R.src_cap = (int)(res_src_lds(s, r) / sizeof(double2));
     const FusedArgs A = make_args(s, 0, 0);
     const Geo g = s->geo();
     while (count > 0) {

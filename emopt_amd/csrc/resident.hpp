@@ -49,6 +49,7 @@ struct ResArgs {
     const SrcBlk *blk;
     int nsrc;
     int ub[6];                        // union box of the sources (PassSrc::ub)
+    int src_cap;                      // deep boxes: double2 of LDS for source values
     double fac[RES_STEPS][6];         // per step: sin t, cos t, env(t) of the H and E halves
 };
 
@@ -70,6 +71,15 @@ constexpr int res_items(bool deep) { return deep ? 2 : 1; }
 // of both do not fit, and the E coefficients live in LDS, where the registers are full
 constexpr bool res_share(int nz, bool deep) { return deep || nz > 4; }
 constexpr bool res_tight(int nz, bool deep) { return !deep && nz > 4; }
+
+// Whether the kernel keeps source values in LDS: the deep one of real eps.
+// From memory, the box that holds a source waited for every plane of the column
+// in turn, twice a step, and all other boxes for it (180x60x80, us a step:
+// one source plane 25 -> 20, the six faces of an adjoint source 38 -> 26).
+// With few planes the waits are few, and the longer code costs 2 to 6 %
+// (126x51x64 39.1 -> 41.8 ms a solve); with complex eps it costs registers that
+// the deep kernel spills (173x101x67 29.2 -> 29.9 ms).
+constexpr bool res_src_in_lds(bool deep, bool ceps) { return deep && !ceps; }
 
 constexpr size_t res_lds(int nz, bool deep, int bx, int by)
 {
@@ -425,13 +435,70 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
 
     const bool anysrc = R.nsrc > 0 && x0 < R.ub[5] && x0 + xw > R.ub[4] && y0 < R.ub[3] &&
                         y0 + yw > R.ub[2] && z0 < R.ub[1] && z0 + zw > R.ub[0];
-    // add(q, value of the block's components c0 .. c0 + 2) for every source cell of the column
-    auto sources = [&](int c0, double st, double ct, double env, auto &&add) {
+    // The box's part of a block: its corner, extent and place in the LDS list, where
+    // the values wait times the factor of the update they enter (6 n double2,
+    // component by component; as many blocks as src_cap holds).
+    constexpr bool LSRC = res_src_in_lds(DEEP, CEPS);
+    double2 *const sl = reinterpret_cast<double2 *>(fac + 6 * RES_STEPS);
+    struct Part { int k, j, i, K, J, I, n; };
+    auto part = [&](const SrcBlk &b, Part &t) {
+        t.k = max(b.k0, x0); t.j = max(b.j0, y0); t.i = max(b.i0, z0);
+        t.K = min(b.k0 + b.K, x0 + xw) - t.k;
+        t.J = min(b.j0 + b.J, y0 + yw) - t.j;
+        t.I = min(b.i0 + b.I, z0 + zw) - t.i;
+        t.n = t.K > 0 && t.J > 0 && t.I > 0 ? t.K * t.J * t.I : 0;
+        return t.n > 0;
+    };
+    if (LSRC && anysrc) {
+        int base = 0;
+        for (int s = 0; s < R.nsrc; ++s) {
+            const SrcBlk sb = src_blk(R.blk, s);
+            Part t;
+            if (!part(sb, t) || base + 6 * t.n > R.src_cap) continue;
+            for (int e = p; e < t.n; e += nt) {
+                const int i = t.i + e / (t.J * t.K), jj = t.j + e / t.K % t.J, kk = t.k + e % t.K;
+                long long m;
+                in_box(sb, i, jj, kk, m);
+                const unsigned c = (((unsigned)i * (unsigned)Ny + (unsigned)jj) * (unsigned)Nx + (unsigned)kk) * 8u;
+#pragma unroll
+                for (int f = 0; f < 6; ++f) {
+                    const double w = f < 3 ? ldo(A.bE, c + (unsigned)f * cs)
+                                           : (MU ? ldo(A.mH, c + (unsigned)(f - 3) * cs) : A.m_s);
+                    double2 v = ld2(sb.f[f] + m);
+                    v.x *= w; v.y *= w;
+                    sl[base + f * t.n + e] = v;
+                }
+            }
+            base += 6 * t.n;
+        }
+    }
+    // for every source cell of the column: put(q, value times factor) of those in
+    // LDS, add(q, value) of the others, of the block's components c0 .. c0 + 2
+    auto sources = [&](int c0, double st, double ct, double env, auto &&put, auto &&add) {
+        int base = 0;
         for (int s = 0; s < R.nsrc; ++s) {
             const SrcBlk sb = src_blk(R.blk, s);
             if (sb.k0 >= x0 + xw || sb.k0 + sb.K <= x0 || sb.j0 >= y0 + yw ||
                 sb.j0 + sb.J <= y0 || sb.i0 >= z0 + zw || sb.i0 + sb.I <= z0)
                 continue;
+            Part t;
+            if (LSRC) part(sb, t);
+            if (LSRC && base + 6 * t.n <= R.src_cap) {
+                const int a = k - t.k, b = j - t.j, zs = t.i - z0, ze = zs + t.I;
+                if (on && (unsigned)a < (unsigned)t.K && (unsigned)b < (unsigned)t.J) {
+                    const double2 *v = sl + base + c0 * t.n + b * t.K + a;
+#pragma unroll
+                    for (int q = 0; q < NZ; ++q)
+                        if (q >= zs && q < ze) {
+                            const double2 *w = v + (q - zs) * t.J * t.K;
+                            const double2 vx = w[0], vy = w[t.n], vz = w[2 * t.n];
+                            put(q, env * (st * vx.x + ct * vx.y), env * (st * vy.x + ct * vy.y),
+                                env * (st * vz.x + ct * vz.y));
+                        }
+                }
+                base += 6 * t.n;
+                continue;
+            }
 #pragma unroll
             for (int q = 0; q < NZ; ++q) {
                 long long m;
@@ -610,6 +677,7 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
             }
             if (anysrc)
                 sources(3, fac[6 * s], fac[6 * s + 1], fac[6 * s + 2],
+                        [&](int q, double vx, double vy, double vz) { hx[q] += vx; hy[q] += vy; hz[q] += vz; },
                         [&](int q, double vx, double vy, double vz) {
                             hx[q] += vx * (MU ? m0[MU ? q : 0] : A.m_s);
                             hy[q] += vy * (MU ? m1[MU ? q : 0] : A.m_s);
@@ -679,6 +747,7 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
             if (anysrc) {
                 const double ix = 1.0 / rx, iy = 1.0 / ry, iz = 1.0 / rz;
                 sources(0, fac[6 * s + 3], fac[6 * s + 4], fac[6 * s + 5],
+                        [&](int q, double vx, double vy, double vz) { ex[q] -= vx; ey[q] -= vy; ez[q] -= vz; },
                         [&](int q, double vx, double vy, double vz) {
                             ex[q] -= vx * (coef(b0, 0, q) * iz);
                             ey[q] -= vy * (coef(b1, 1, q) * ix);
