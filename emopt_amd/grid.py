@@ -465,8 +465,8 @@ _LIMIT_MSG = ("a cell meets more than %d primitives or %d polygon edges "
 
 
 def _cell_exact(order, xa, xb, ya, yb, bg):
-    """One cell by the reference's rule, the operations of k_mat_inplane
-    (ss == 0) in the same order; order = the rings' corner flags
+    """One cell by the reference's rule, the operations of k_mat_exact
+    in the same order; order = the rings' corner flags
     (c1, c2, c3, c4) in priority order."""
     A = (xb - xa) * (yb - ya)
     rem = A
