@@ -211,25 +211,26 @@ def boundary_deps(sim, eps, prim, velocity, tol=0.0):
                       min(Nx, int(np.ceil(ex1 / dx - sx + 0.5)) + 2),
                       max(0, int(np.floor(ey0 / dy - sy - 0.5)) - 1),
                       min(Ny, int(np.ceil(ey1 / dy - sy + 0.5)) + 2)))
-    # the z segments the primitive is in, and their rings in priority order
+    # the z segments the primitive is in, with their entries in priority order and
+    # the moving one's place among them (the last, where it was added more than once)
     segs = []
     for za, zb in zip(bounds[:-1], bounds[1:]):
         if not (entry[1] <= za and entry[2] >= zb):
             continue
         active = sorted([e for e in active_all if e[1] <= za and e[2] >= zb],
                         key=lambda e: (e[0].layer, e[3]))
-        segs.append((za, zb, active))
+        segs.append((za, zb, active, max(n for n, e in enumerate(active) if e[0] is prim)))
     ring_of = {}
-    for _, _, active in segs:
+    for _, _, active, _ in segs:
         for e in active:
             if id(e) not in ring_of:
                 ring_of[id(e)] = eps._ring(e[0])
     if getattr(sim, "_h", None) is not None:
-        inplane = _inplane_device(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg)
+        inplane = _inplane_device(sim, segs, ring_of, edges, boxes, dx, dy, bg)
     else:
         inplane = None
     if inplane is None:
-        inplane = _inplane_host(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg,
+        inplane = _inplane_host(sim, segs, ring_of, edges, boxes, dx, dy, bg,
                                 (ex0, ex1, ey0, ey1))
     comps, cells, vals = [], [], []
     for c, (_, _, sz) in enumerate(sim.YEE_SHIFTS[:3]):
@@ -237,7 +238,7 @@ def boundary_deps(sim, eps, prim, velocity, tol=0.0):
         zlo, zhi = zc - dz / 2, zc + dz / 2
         k1, k2, j1, j2 = boxes[c]
         cell, val = [], []
-        for (za, zb, _), d2 in zip(segs, inplane[c]):
+        for (za, zb, _, _), d2 in zip(segs, inplane[c]):
             fz = np.clip(np.minimum(zhi, zb) - np.maximum(zlo, za), 0, None) / dz
             iz = np.nonzero(fz > 0)[0]
             j, k = np.nonzero(d2)
@@ -263,16 +264,15 @@ def boundary_deps(sim, eps, prim, velocity, tol=0.0):
     return np.concatenate(comps), np.concatenate(cells), np.concatenate(vals)
 
 
-def _inplane_host(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg, extent):
+def _inplane_host(sim, segs, ring_of, edges, boxes, dx, dy, bg, extent):
     """In-plane derivatives [component][segment][j, k] of the boxes' cells."""
     ex0, ex1, ey0, ey1 = extent
     res = []
     for c, (sx, sy, _) in enumerate(sim.YEE_SHIFTS[:3]):
         k1, k2, j1, j2 = boxes[c]
         per = []
-        for _, _, active in segs:
+        for _, _, active, p in segs:
             rings = [ring_of[id(e)] for e in active]
-            p = next(n for n, e in enumerate(active) if e[0] is prim)
             d2 = np.zeros((max(0, j2 - j1), max(0, k2 - k1)), dtype=np.complex128)
             for j in range(j1, j2):
                 yc = (j + sy) * dy
@@ -290,19 +290,18 @@ def _inplane_host(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg, extent):
     return res
 
 
-def _inplane_device(sim, segs, ring_of, prim, edges, boxes, dx, dy, bg):
+def _inplane_device(sim, segs, ring_of, edges, boxes, dx, dy, bg):
     """_inplane_host on the solver's GPU (emf_shape_deps), the same doubles;
     None where a cell counts more primitives than the device holds."""
     ids, rings = {}, []
     off, lst, mine = [0], [], []
-    for _, _, active in segs:
-        for n, e in enumerate(active):
+    for _, _, active, p in segs:
+        for e in active:
             if id(e) not in ids:
                 ids[id(e)] = len(rings)
                 rings.append(ring_of[id(e)])
             lst.append(ids[id(e)])
-            if e[0] is prim:
-                mine.append(n)
+        mine.append(p)
         off.append(len(lst))
     if not segs:
         return [[], [], []]
