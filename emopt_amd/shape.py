@@ -213,18 +213,17 @@ def boundary_deps(sim, eps, prim, velocity, tol=0.0):
                       min(Ny, int(np.ceil(ey1 / dy - sy + 0.5)) + 2)))
     # the z segments the primitive is in, with their entries in priority order and
     # the moving one's place among them (the last, where it was added more than once)
-    segs = []
+    segs, ring_of = [], {}
     for za, zb in zip(bounds[:-1], bounds[1:]):
         if not (entry[1] <= za and entry[2] >= zb):
             continue
         active = sorted([e for e in active_all if e[1] <= za and e[2] >= zb],
                         key=lambda e: (e[0].layer, e[3]))
-        segs.append((za, zb, active, max(n for n, e in enumerate(active) if e[0] is prim)))
-    ring_of = {}
-    for _, _, active, _ in segs:
         for e in active:
             if id(e) not in ring_of:
                 ring_of[id(e)] = eps._ring(e[0])
+        active = [e for e in active if ring_of[id(e)] is not None]   # nothing left of it
+        segs.append((za, zb, active, max(n for n, e in enumerate(active) if e[0] is prim)))
     if getattr(sim, "_h", None) is not None:
         inplane = _inplane_device(sim, segs, ring_of, edges, boxes, dx, dy, bg)
     else:

@@ -1,10 +1,11 @@
 """boundary_deps on structured materials whose entries are not one per primitive
-(CPU only): an object added twice.  The lists that go to the device are checked
-with a stand-in library."""
+(CPU only): an object added twice, polygons with nothing left of them.  The
+lists that go to the device are checked with a stand-in library."""
 import ctypes
 import types
 
 import numpy as np
+import pytest
 
 from emopt_amd import grid
 from emopt_amd.shape import boundary_deps, rect_edge_velocity
@@ -77,3 +78,25 @@ def test_moving_object_added_twice_host_rule():
         want += _dense(boundary_deps(host, part, mine, rect_edge_velocity("xr")))
     assert np.abs(want).max() > 0
     np.testing.assert_allclose(got, want, rtol=0, atol=1e-12 * np.abs(want).max())
+
+
+@pytest.mark.parametrize("device", [False, True])
+def test_polygons_with_nothing_left_do_not_count(device):
+    """A polygon of fewer than three vertices is no ring: the derivative is that
+    without it, whichever of them comes first."""
+    host, dev = _sims()
+    res = []
+    for empty in (False, True):
+        eps = grid.StructuredMaterial3D(N[0] * D, N[1] * D, N[2] * D, D, D, D)
+        p = grid.Rectangle(1.0, 0.8, 0.73, 0.55, material_value=9.0, layer=2)
+        if empty:
+            for layer in (1, 3):
+                g = grid.Polygon([0.2, 0.9, 0.5], [0.2, 0.3, 0.9], material_value=4.0, layer=layer)
+                g.xs, g.ys = g.xs[:2], g.ys[:2]
+                eps.add_primitive(g, 0.0, 1.2)
+        eps.add_primitive(p, 0.0, 1.2)
+        res.append(boundary_deps(dev if device else host, eps, p, rect_edge_velocity("xr")))
+        if device:
+            assert dev._lib.mine == [0]
+    for a, b in zip(*res):
+        assert len(a) > 0 and np.array_equal(a, b)
