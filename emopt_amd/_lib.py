@@ -20,8 +20,15 @@ import numpy as np
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libemfdtd.so")
 
 
+ERR_ARG, ERR_HIP, ERR_NOMEM, ERR_STATE = -1, -2, -3, -4     # EMF_ERR_* of include/emfdtd.h
+
+
 class EmfError(RuntimeError):
-    """A libemfdtd call returned a non-zero status."""
+    """A libemfdtd call returned a non-zero status (``code``)."""
+
+    def __init__(self, msg, code=None):
+        super().__init__(msg)
+        self.code = code
 
 
 class SolveInfo(ctypes.Structure):
@@ -151,7 +158,7 @@ class _Checked:
             rc = fn(*args)
             if rc < 0 or (rc != 0 and name not in _COUNT_RESULT):
                 msg = raw.emf_last_error()
-                raise EmfError("%s failed (%d): %s" % (name, rc, msg.decode() if msg else ""))
+                raise EmfError("%s failed (%d): %s" % (name, rc, msg.decode() if msg else ""), rc)
             return rc
 
         call.__name__ = name

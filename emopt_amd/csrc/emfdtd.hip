@@ -3062,7 +3062,12 @@ int emf_shape_deps(emf_solver *s, const emf_prim *rings, int nrings, const doubl
                    const double *edges, int nedges, const int *box, const double *shifts,
                    double *out, int *limit)
 {
-    LOCK(s);
+    if (!s) EMF_FAIL(EMF_ERR_ARG, "null solver handle");
+    // not waited for: the caller's own rule takes less than a solve in another thread
+    std::unique_lock<std::mutex> lk(s->mtx, std::try_to_lock);
+    if (!lk.owns_lock() || s->in_batch)
+        EMF_FAIL(EMF_ERR_STATE, "handle is solving or a member of a batch");
+    if (hipSetDevice(s->dev) != hipSuccess) EMF_FAIL(EMF_ERR_HIP, "hipSetDevice(%d) failed", s->dev);
     if (!seg_off || !seg_ring || !seg_p || !edges || !box || !shifts || !out || !limit || nseg < 1 ||
         nedges < 1)
         EMF_FAIL(EMF_ERR_ARG, "bad arguments");

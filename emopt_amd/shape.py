@@ -44,6 +44,7 @@ from ctypes import byref, c_int
 
 import numpy as np
 
+from ._lib import ERR_NOMEM, ERR_STATE, EmfError
 from .grid import Ellipse, Polygon, Rectangle, StructuredMaterial3D
 
 __all__ = ["boundary_deps", "rect_edge_velocity", "polygon_vertex_velocity"]
@@ -291,7 +292,9 @@ def _inplane_host(sim, segs, ring_of, edges, boxes, dx, dy, bg, extent):
 
 def _inplane_device(sim, segs, ring_of, edges, boxes, dx, dy, bg):
     """_inplane_host on the solver's GPU (emf_shape_deps), the same doubles;
-    None where a cell counts more primitives than the device holds."""
+    None where the host has to: a cell counts more primitives than the device
+    holds, the solver is busy (a batch member, or solving in another thread), or
+    the device has no room."""
     ids, rings = {}, []
     off, lst, mine = [0], [], []
     for _, _, active, p in segs:
@@ -322,10 +325,15 @@ def _inplane_device(sim, segs, ring_of, edges, boxes, dx, dy, bg):
     out = np.zeros(sum(int(np.prod(s)) for s in shape), dtype=np.complex128)
     off, lst, mine = (np.array(v, dtype=np.int32) for v in (off, lst, mine))
     limit = c_int(0)
-    sim._lib.emf_shape_deps(sim._h, recs.ctypes.data, len(recs), vx.ctypes.data, vy.ctypes.data, nv,
-                            dx, dy, bg.real, bg.imag, off.ctypes.data, lst.ctypes.data,
-                            mine.ctypes.data, len(segs), ed.ctypes.data, len(ed), box.ctypes.data,
-                            sh.ctypes.data, out.ctypes.data, byref(limit))
+    try:
+        sim._lib.emf_shape_deps(sim._h, recs.ctypes.data, len(recs), vx.ctypes.data, vy.ctypes.data,
+                                nv, dx, dy, bg.real, bg.imag, off.ctypes.data, lst.ctypes.data,
+                                mine.ctypes.data, len(segs), ed.ctypes.data, len(ed),
+                                box.ctypes.data, sh.ctypes.data, out.ctypes.data, byref(limit))
+    except EmfError as exc:
+        if exc.code not in (ERR_STATE, ERR_NOMEM):
+            raise
+        return None
     if limit.value:
         return None
     res, at = [], 0

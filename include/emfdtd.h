@@ -481,7 +481,8 @@ EMF_API int emf_build_structured(emf_solver *s, const emf_prim *prims, int nprim
  * y1, length, normal velocity at either end.  box: k1, k2, j1, j2 per eps
  * component, shifts its in-cell offset (x, y).  out: complex, per component
  * [segment][j][k].  *limit: nonzero when a cell counts more primitives than the
- * device holds; out is then incomplete. */
+ * device holds; out is then incomplete.  A handle that is a batch member or in
+ * use by another thread is refused (EMF_ERR_STATE), not waited for. */
 EMF_API int emf_shape_deps(emf_solver *s, const emf_prim *rings, int nrings, const double *vx,
                            const double *vy, int nverts, double dx, double dy, double bg_re,
                            double bg_im, const int *seg_off, const int *seg_ring, const int *seg_p,

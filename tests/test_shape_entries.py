@@ -1,13 +1,14 @@
 """boundary_deps on structured materials whose entries are not one per primitive
-(CPU only): an object added twice, polygons with nothing left of them.  The
-lists that go to the device are checked with a stand-in library."""
+(CPU only): an object added twice, polygons with nothing left of them, and on
+solvers that cannot take the call.  The lists that go to the device are checked
+with a stand-in library."""
 import ctypes
 import types
 
 import numpy as np
 import pytest
 
-from emopt_amd import grid
+from emopt_amd import _lib, grid
 from emopt_amd.shape import boundary_deps, rect_edge_velocity
 
 SHIFTS = ((0.5, 0.0, -0.5), (0.0, 0.5, -0.5), (0.0, 0.0, 0.0))
@@ -100,3 +101,22 @@ def test_polygons_with_nothing_left_do_not_count(device):
             assert dev._lib.mine == [0]
     for a, b in zip(*res):
         assert len(a) > 0 and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("code", [_lib.ERR_STATE, _lib.ERR_NOMEM, _lib.ERR_HIP])
+def test_refused_by_the_solver(code):
+    """A solver that is a batch member or busy, or a device without room, leaves
+    the derivative to the host; other errors are raised."""
+    eps, p = _twice()
+    host, dev = _sims()
+
+    def refuse(*args):
+        raise _lib.EmfError("refused", code)
+    dev._lib.emf_shape_deps = refuse
+    if code == _lib.ERR_HIP:
+        with pytest.raises(_lib.EmfError):
+            boundary_deps(dev, eps, p, rect_edge_velocity("xr"))
+        return
+    for a, b in zip(boundary_deps(dev, eps, p, rect_edge_velocity("xr")),
+                    boundary_deps(host, eps, p, rect_edge_velocity("xr"))):
+        assert np.array_equal(a, b)
