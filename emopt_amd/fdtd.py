@@ -740,6 +740,12 @@ class FDTD(MaxwellSolver):
         pidx = np.asarray(pidx, dtype=np.int32)
         comp, cell = np.asarray(comp, dtype=np.int32), np.asarray(cell, dtype=np.int64)
         deps = np.asarray(deps, dtype=np.complex128)
+        if pidx.ndim != 1:
+            raise ValueError("pidx must be one-dimensional")
+        n = len(pidx)
+        for name, a in (("comp", comp), ("cell", cell), ("deps", deps)):
+            if a.ndim == 0 or min(len(a), a.size) < n:     # n of each are read
+                raise IndexError("%s of shape %s for %d entries" % (name, a.shape, n))
         if np.any(pidx[1:] < pidx[:-1]):       # group by parameter
             order = np.argsort(pidx, kind="stable")
             pidx, comp, cell, deps = pidx[order], comp[order], cell[order], deps[order]
