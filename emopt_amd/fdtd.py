@@ -295,9 +295,11 @@ class FDTD(MaxwellSolver):
         that replaces them is asked for its arrays instead."""
         return (isinstance(self._eps, StructuredMaterial3D) and self._eps.stock_samplers()
                 and type(self._mu) is ConstantMaterial3D
+                and getattr(self._mu.get_values, "__func__", None) is ConstantMaterial3D.get_values
                 and math.isfinite(self._mu.material_value.real)
-                and type(self)._sample is FDTD._sample
-                and type(self).set_material_arrays is FDTD.set_material_arrays)
+                and getattr(self._sample, "__func__", None) is FDTD._sample
+                and getattr(self.set_material_arrays, "__func__", None)
+                is FDTD.set_material_arrays)
 
     def _sample(self, m, k1, k2, j1, j2, i1, i2, sx, sy, sz, arr=None):
         """Material values of a box at one Yee offset: structured materials
