@@ -8,9 +8,10 @@ itself (``emf_time_steps``), on its own grid, materials and CPML, and the
 fastest is kept.  Every candidate computes bit-for-bit the same fields (the
 parity tests check each one), so tuning never changes results.  Winners are
 cached per (grid, complex eps, uniform mu) in memory and, when a path is given,
-in a JSON file.  Where solves run resident (emf_resident; 3 to 5 times faster
-than any step kernel) a winner of another kind than the two passes is reported
-but not applied, which leaves them so.
+in a JSON file.  Where solves run resident (emf_resident), which is faster than
+any step kernel, a winner of another kind than the two passes, which would end
+that, is reported but not applied: the fastest of the two passes' shapes is (from
+the cache, the solver keeps its own).
 
 Batches: steps per graph replay, z planes per work-group and persistent
 work-groups per CU are timed on a sample of the batch's members (a fixed
@@ -50,13 +51,11 @@ def _load(path):
     return {}
 
 
-def _apply(L, h, best):
-    """Select the step kernel `best`, unless that ends resident solves."""
+def _resident(L, h):
+    """Whether the solver's next solve would run resident."""
     boxes = ctypes.c_int()
-    L.emf_set_tuning(h, *SOLVE_CANDIDATES[0])
     L.emf_resident(h, ctypes.byref(boxes))
-    if boxes.value == 0 or best[0] == 1:
-        L.emf_set_tuning(h, *best)
+    return boxes.value > 0
 
 
 def tune_solver(sim, candidates=None, steps=40, warmup=8, cache_path=None, verbose=False):
@@ -67,14 +66,14 @@ def tune_solver(sim, candidates=None, steps=40, warmup=8, cache_path=None, verbo
     disk = _load(cache_path)
     if key in _cache or key in disk:
         best = tuple(_cache.get(key) or disk[key])
-        if not sim._mats_ready:
-            sim.build()
-        _apply(sim._lib, sim._h, best)
+        if best[0] == 1 or not _resident(sim._lib, sim._h):
+            sim._lib.emf_set_tuning(sim._h, *best)
         return best, {}
     if not sim._mats_ready:
         sim.build()
     sim._register(sim._sources)
     L, h = sim._lib, sim._h
+    resident = _resident(L, h)
     times = {}
     out = np.zeros(3)
     for cand in candidates or SOLVE_CANDIDATES:
@@ -90,7 +89,10 @@ def tune_solver(sim, candidates=None, steps=40, warmup=8, cache_path=None, verbo
         if verbose:
             print("tune %s: %.4f ms/step" % (cand, times[cand]))
     best = min(times, key=times.get)
-    _apply(L, h, best)
+    use = best
+    if resident and best[0] != 1:
+        use = min((c for c in times if c[0] == 1), key=times.get, default=SOLVE_CANDIDATES[0])
+    L.emf_set_tuning(h, *use)
     L.emf_reset_pml(h)
     L.emf_zero_fields(h)
     _cache[key] = list(best)

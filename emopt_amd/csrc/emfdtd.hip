@@ -1114,7 +1114,8 @@ bool res_split(const emf_solver *s, int GX, int GY, int GZ, ResPlan &r)
 // 64x64x64 and 25.8 on 120x80x60.
 bool resident_plan(const emf_solver *s, int ncu, ResPlan &best)
 {
-    if (s->res_off || s->kind != 1 || s->wide || s->Nx < 2 || s->Ny < 2 || s->Nz < 2) return false;
+    if (s->res_off || s->kind != 1 || s->wide || s->wide_force || s->Nx < 2 || s->Ny < 2 || s->Nz < 2)
+        return false;
     double bt = 1e30;
     for (int GZ = 1; GZ <= std::min(ncu, s->Nz); ++GZ) {
         if ((s->Nz + GZ - 1) / GZ > res_planes_deep(!s->mu_uniform)) continue;
@@ -2857,7 +2858,9 @@ int emf_resident(emf_solver *s, int *boxes)
 {
     LOCK(s);
     if (!boxes) EMF_FAIL(EMF_ERR_ARG, "null output");
-    CHECK(check_ready(s));
+    // before the materials are set: for eps as declared (emf_set_complex_eps) and a uniform mu
+    if (s->mat_set) CHECK(check_ready(s));
+    else if (s->Nx <= 0 || s->Ny <= 0 || s->Nz <= 0) EMF_FAIL(EMF_ERR_STATE, "grid dims not set");
     ResPlan plan;
     int ncu = 0;
     CHECK(res_cus(s->dev, &ncu));

@@ -385,7 +385,8 @@ EMF_API int emf_set_wide_offsets(emf_solver *s, int force);
 EMF_API int emf_set_resident(emf_solver *s, int on, int spin);
 
 /* *boxes = work-groups of the resident launches this solver's next emf_solve
- * would use, 0 where it uses the step kernels. */
+ * would use, 0 where it uses the step kernels.  Before the materials are set:
+ * the answer for a uniform mu. */
 EMF_API int emf_resident(emf_solver *s, int *boxes);
 
 /* Work-group shape of the H pass of the two-pass kernels (kinds 1 and 3):
