@@ -28,6 +28,7 @@
 
 #include "../../include/emfdtd.h"
 #include "batch.hpp"
+#include "per_device.hpp"
 #include "resident.hpp"
 #include "material.hpp"
 #include "shape.hpp"
@@ -1218,10 +1219,11 @@ int res_launch_t(emf_solver *s, const ResPlan &r, const ResArgs &R, const FusedA
                  const Geo &g, const int *done)
 {
     auto K = k_resident<NZ, CE, MU>;
-    static std::atomic<bool> lds_set{ false };
-    if (!lds_set.exchange(true))
-        HIPCHK(hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kResLds));
+    static OncePerDevice lds_set;
+    HIPCHK((hipError_t)lds_set.run(s->dev, [&] {
+        return (int)hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)kResLds);
+    }));
     hipLaunchKernelGGL(K, dim3(r.boxes()), dim3(r.threads), r.lds + (size_t)R.src_cap * sizeof(double2),
                        s->stream, R, A, g, done);
     HIPCHK(hipGetLastError());
