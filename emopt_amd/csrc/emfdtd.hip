@@ -1131,45 +1131,15 @@ bool resident_plan(const emf_solver *s, int ncu, ResPlan &best)
     return bt < 1e30;
 }
 
-// Work-groups of resident launches in flight on a device: all of them have to
-// be able to run at once, so no more than the CUs are admitted together.
-struct ResGate {
-    std::mutex m;
-    std::condition_variable cv;
-    int used = 0, ncu = 0;
-};
-ResGate g_res_gate[64];
-
-struct ResHold {
-    ResGate *g = nullptr;
-    int n = 0;
-    void take(ResGate &gate, int boxes)
-    {
-        std::unique_lock<std::mutex> lk(gate.m);
-        gate.cv.wait(lk, [&] { return gate.used + boxes <= gate.ncu; });
-        gate.used += boxes;
-        g = &gate;
-        n = boxes;
-    }
-    void give()
-    {
-        if (!g) return;
-        { std::lock_guard<std::mutex> lk(g->m); g->used -= n; }
-        g->cv.notify_all();
-        g = nullptr;
-    }
-    ~ResHold() { give(); }
-};
+ResGate g_res_gate[PER_DEVICE_MAX];
 
 int res_cus(int dev, int *ncu)
 {
     *ncu = 0;
-    if (dev < 0 || dev >= 64) return EMF_OK;
-    ResGate &gate = g_res_gate[dev];
-    std::lock_guard<std::mutex> lk(gate.m);
-    if (!gate.ncu)
-        HIPCHK(hipDeviceGetAttribute(&gate.ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    *ncu = gate.ncu;
+    if (dev < 0 || dev >= PER_DEVICE_MAX) return EMF_OK;
+    HIPCHK((hipError_t)g_res_gate[dev].cus(ncu, [&](int *n) {
+        return (int)hipDeviceGetAttribute(n, hipDeviceAttributeMultiprocessorCount, dev);
+    }));
     return EMF_OK;
 }
 

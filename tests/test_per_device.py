@@ -63,3 +63,42 @@ int main()
     return 0;
 }
 """)
+
+
+def test_gate_counts_work_groups_by_xcd_and_admits_in_order(tmp_path):
+    _run(tmp_path, """
+using ms = std::chrono::milliseconds;
+int main()
+{
+    ResGate g;
+    int n = 0;
+    EXPECT(g.cus(&n, [](int *v) { *v = 256; return 3; }) == 3 && n == 0);
+    EXPECT(g.cus(&n, [](int *v) { *v = 256; return 0; }) == 0 && n == 256);
+    EXPECT(g.cus(&n, [](int *v) { *v = 1; return 0; }) == 0 && n == 256);
+    // 100 + 156 = 256, but 13 + 20 CUs of the first XCDs
+    ResHold a;
+    a.take(g, 100);
+    std::atomic<int> order{ 0 };
+    int b_at = 0, c_at = 0;
+    std::thread tb([&] { ResHold h; h.take(g, 156); b_at = ++order; });
+    std::this_thread::sleep_for(ms(100));
+    // 8 would fit beside the first, but came after
+    std::thread tc([&] { ResHold h; h.take(g, 8); c_at = ++order; });
+    std::this_thread::sleep_for(ms(100));
+    EXPECT(order == 0);
+    a.give();
+    tb.join(); tc.join();
+    EXPECT(b_at == 1 && c_at == 2);
+    // 96 + 160 fit side by side
+    ResHold d, e;
+    d.take(g, 96);
+    e.take(g, 160);
+    d.give(); e.give();
+    // alone, all of them, also where the CUs are no multiple of the XCDs
+    ResGate odd;
+    odd.cus(&n, [](int *v) { *v = 20; return 0; });
+    ResHold f;
+    f.take(odd, 20);
+    return 0;
+}
+""")
