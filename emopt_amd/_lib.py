@@ -118,6 +118,7 @@ _SIGS = {
     "emf_set_wide_offsets": ([_P, c_int], c_int),
     "emf_set_resident": ([_P, c_int, c_int], c_int),
     "emf_resident": ([_P, POINTER(c_int)], c_int),
+    "emf_resident_stalls": ([_P, POINTER(c_int)], c_int),
     "emf_field_products": ([_P, c_int] + [c_int] * 6 + [_P], c_int),
     "emf_stage_clear": ([_P], c_int),
     "emf_stage_count": ([_P, _P], c_int),

@@ -469,7 +469,7 @@ int emf_batch_add(emf_batch *b, emf_solver *s, int slot, double rtol, double nma
     q.t_add = std::chrono::steady_clock::now();
     q.rtol = rtol; q.nmax = nmax; q.Tn = Tn; q.fixed_n0 = fixed_n0;
     // a member that fits on chip waits for its own resident solve (emf_batch_run)
-    const int rc = resident_plan(s, ncu, plan) ? solve_prepare(s, nmax, Tn) : batch_tile(b, id);
+    const int rc = resident_next(s, ncu, plan) ? solve_prepare(s, nmax, Tn) : batch_tile(b, id);
     if (rc != EMF_OK) {
         dfree(q.fac);
         q = BatchSlot{};

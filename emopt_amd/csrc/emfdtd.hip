@@ -228,8 +228,11 @@ struct emf_solver {
     double2 *scratch = nullptr;
     size_t scratch_n = 0;
 
-    // resident steps (resident.hpp): off once a launch stalled, or by emf_set_resident
+    // resident steps (resident.hpp): off by emf_set_resident; after a stall the next
+    // res_skip solves leave them out
     bool res_off = false;
+    int res_skip = 0, res_row = 0;       // res_row: stalls since a resident solve went through
+    int res_stalls = 0;
     int res_spin = RES_SPIN;
     unsigned long long *res_halo = nullptr;
     size_t res_halo_n = 0;
@@ -1115,7 +1118,7 @@ bool res_split(const emf_solver *s, int GX, int GY, int GZ, ResPlan &r)
 // 64x64x64 and 25.8 on 120x80x60.
 bool resident_plan(const emf_solver *s, int ncu, ResPlan &best)
 {
-    if (s->res_off || s->kind != 1 || s->wide || s->wide_force || s->Nx < 2 || s->Ny < 2 || s->Nz < 2)
+    if (s->res_off || s->res_skip > 0 || s->kind != 1 || s->wide || s->wide_force || s->Nx < 2 || s->Ny < 2 || s->Nz < 2)
         return false;
     double bt = 1e30;
     for (int GZ = 1; GZ <= std::min(ncu, s->Nz); ++GZ) {
@@ -1129,6 +1132,27 @@ bool resident_plan(const emf_solver *s, int ncu, ResPlan &best)
             }
     }
     return bt < 1e30;
+}
+
+// The plan of the solve that starts now: as resident_plan, and a solve that is to
+// leave resident steps out after a stall counts as done.
+bool resident_next(emf_solver *s, int ncu, ResPlan &r)
+{
+    if (resident_plan(s, ncu, r)) return true;
+    if (s->res_skip > 0) --s->res_skip;
+    return false;
+}
+
+// A launch stalled: something else held CUs of the device for seconds.  The next
+// solve takes the passes, and with every further stall in a row twice as many,
+// up to 64: one that stalls loses the polls' seconds, one that goes through
+// gains a few times its own time.
+void resident_stalled(emf_solver *s)
+{
+    s->res_skip = 1 << std::min(s->res_row, 6);
+    ++s->res_row;
+    ++s->res_stalls;
+    s->res_halo_clean = false;
 }
 
 ResGate g_res_gate[PER_DEVICE_MAX];
@@ -1428,7 +1452,7 @@ int solve_any(emf_solver *s, int slot, double rtol, double nmax, long long Tn, l
     ResPlan plan;
     int ncu = 0;
     CHECK(res_cus(s->dev, &ncu));
-    if (resident_plan(s, ncu, plan)) {
+    if (resident_next(s, ncu, plan)) {
         ResHold hold;
         hold.take(g_res_gate[s->dev], plan.boxes());
         const int rc = solve_run(s, slot, rtol, nmax, Tn, fixed_n0, &plan, run);
@@ -1437,9 +1461,10 @@ int solve_any(emf_solver *s, int slot, double rtol, double nmax, long long Tn, l
         CHECK(rc);
         if (run.stalled) {
             // the work-groups of a launch did not run together: from the start with the passes
-            s->res_off = true;
-            s->res_halo_clean = false;
+            resident_stalled(s);
             CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
+        } else {
+            s->res_row = 0;
         }
     } else {
         CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
@@ -2822,6 +2847,7 @@ int emf_set_resident(emf_solver *s, int on, int spin)
     LOCK(s);
     if ((on != 0 && on != 1) || spin < 0) EMF_FAIL(EMF_ERR_ARG, "on must be 0 or 1, spin >= 0");
     s->res_off = !on;
+    s->res_skip = s->res_row = 0;
     s->res_spin = spin > 0 ? spin : RES_SPIN;
     return EMF_OK;
 }
@@ -2837,6 +2863,14 @@ int emf_resident(emf_solver *s, int *boxes)
     int ncu = 0;
     CHECK(res_cus(s->dev, &ncu));
     *boxes = resident_plan(s, ncu, plan) ? plan.boxes() : 0;
+    return EMF_OK;
+}
+
+int emf_resident_stalls(emf_solver *s, int *stalls)
+{
+    LOCK(s);
+    if (!stalls) EMF_FAIL(EMF_ERR_ARG, "null output");
+    *stalls = s->res_stalls;
     return EMF_OK;
 }
 

@@ -118,6 +118,7 @@ class FDTD(MaxwellSolver):
         self._mu = None
         self._mats_ready = False
         self._have = [False, False]    # result slots filled (fwd, adj)
+        self._stalls = 0               # stalled resident launches already reported
         self.forward_count = 0
         self.adjoint_count = 0
         self.fixed_n0 = None           # pin the capture step (parity runs)
@@ -508,6 +509,12 @@ class FDTD(MaxwellSolver):
             warnings.warn("Maximum number of time steps exceeded.")
         if info.status == 3:
             warnings.warn("The fields are not finite (NaN or Inf) at the last convergence check.")
+        stalls = _lib.ctypes.c_int()
+        self._lib.emf_resident_stalls(self._h, _lib.ctypes.byref(stalls))
+        if stalls.value != self._stalls:
+            self._stalls = stalls.value
+            warnings.warn("Other work kept the GPU from running the solve resident; it was "
+                          "repeated with the step kernels.", RuntimeWarning)
         self._have[slot] = True
 
     @property

@@ -379,15 +379,21 @@ EMF_API int emf_set_wide_offsets(emf_solver *s, int force);
  * the chip's registers (up to about 655,000 cells with real eps and uniform
  * mu, 393,000 otherwise) takes many steps per launch with its state on chip.
  * on = 0 keeps such a solve on the step kernels; spin > 0 bounds the polls for
- * a neighbour's data before the launch counts as stalled and the solve is
- * repeated with the step kernels (0: the default, some seconds).  The fields
- * agree to roundoff either way.  No counterpart in the reference. */
+ * a neighbour's data before the launch counts as stalled (something else held
+ * CUs of the device meanwhile) and the solve is repeated with the step kernels
+ * (0: the default, some seconds).  The solve after it takes the step kernels too,
+ * then resident steps are tried again; with further stalls in a row 2, 4, ... 64
+ * solves later.  This call ends such a pause.  The fields agree to roundoff
+ * either way.  No counterpart in the reference. */
 EMF_API int emf_set_resident(emf_solver *s, int on, int spin);
 
 /* *boxes = work-groups of the resident launches this solver's next emf_solve
  * would use, 0 where it uses the step kernels.  Before the materials are set:
  * the answer for a uniform mu. */
 EMF_API int emf_resident(emf_solver *s, int *boxes);
+
+/* *stalls = resident launches of this solver that stalled, in all. */
+EMF_API int emf_resident_stalls(emf_solver *s, int *stalls);
 
 /* Work-group shape of the H pass of the two-pass kernels (kinds 1 and 3):
  * rows (waves) per work-group tyg in {1, 2, 4, 8} and z planes per work-group
