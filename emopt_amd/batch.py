@@ -5,11 +5,12 @@ convergence test; one kernel launch per half step covers all members, and
 every member's solve loop (emopt/fdtd.py:994-1194) runs on the device, so the
 host only replays a captured hipGraph of ``steps_per_graph`` steps and reads
 the members' states between replays.  A member whose grid fits on chip takes
-its own resident solve instead (a few at once where they leave CUs idle), as
-``solve_forward`` does: 5 to 10 us per step of up to 655,000 cells.  Members may
+its own resident solve instead, as ``solve_forward`` does: 5 to 10 us per step of
+up to 655,000 cells.  Members may
 be added while others run (continuous batching).  A member's fields agree with those of
 ``solve_forward`` / ``solve_adjoint`` on the same problem to roundoff (same
-n0 and step counts), and do not depend on the other members.
+n0 and step counts; to the bit where it is resident), and do not depend on the
+other members, nor on how ``run`` was called.
 
     b = Batch()
     ids = [b.add(sim) for sim in sims]          # forward solves

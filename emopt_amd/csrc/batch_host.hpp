@@ -10,7 +10,9 @@
 // memset or copy nodes.
 //
 // A member whose grid fits on chip (resident.hpp) is not stepped by these
-// kernels: a run until members finish gives it its own resident solve.
+// kernels but by its own resident solve loop, in which a replay counts as `spg`
+// steps.  Which of the two a member is, is settled when it is admitted, and its
+// loop's launches do not depend on how the calls divide it.
 //
 // Lanes: the other members are split into cache-sized groups, and `lanes` groups
 // are stepped at once, each by its own stream, copy of the table and graph.
@@ -26,8 +28,7 @@ struct BatchSlot {
     int slot = 0;
     bool finished = false;
     bool tiled = false;                 // stepped by the batch's kernels (else resident, on its own)
-    double rtol = 0, nmax = 0;          // as admitted
-    long long Tn = 0, fixed_n0 = -1;
+    SolveLoop loop;                     // as admitted, and where a resident solve stands
     double *fac = nullptr;              // device per-step factors
     emf_solve_info info{};
     std::chrono::steady_clock::time_point t_add;
@@ -53,6 +54,7 @@ struct emf_batch {
     long long group_bytes = 0;          // hot-state bytes per group (0: one group)
     int rotate = 0;                     // 1: groups take turns; 0: first group until done
     long long next_seq = 0;             // admission counter
+    long long own_due = 0;              // steps that resident members are due (negative: ahead)
     int ncu = 0;
     BTable *T = nullptr;                // one copy of the table per lane
     BMember *M = nullptr;
@@ -210,8 +212,9 @@ int batch_tile(emf_batch *b, int id)
     BatchSlot &q = b->sl[id];
     emf_solver *s = q.s;
     const int slot = q.slot;
-    const long long Tn = q.Tn, fixed_n0 = q.fixed_n0;
-    const long long n_stop = q.nmax < 0 ? 0 : (long long)floor(std::min(q.nmax, 1e15)) + 1;
+    const long long Tn = q.loop.Tn, fixed_n0 = q.loop.fixed_n0;
+    const double nmax = q.loop.nmax;
+    const long long n_stop = nmax < 0 ? 0 : (long long)floor(std::min(nmax, 1e15)) + 1;
     const long long nlast = fixed_n0 >= 0 ? fixed_n0 : n_stop;
     const long long nfac = nlast + 2 * Tn + 1;
     // the solver's state as emf_solve sets it up (emopt/fdtd.py:1016-1018)
@@ -268,8 +271,8 @@ int batch_tile(emf_batch *b, int id)
     B.n_stop = n_stop;
     B.fixed_n0 = fixed_n0;
     B.Tn = Tn;
-    B.amp_rtol = q.rtol;
-    B.phi_rtol = sqrt(q.rtol);
+    B.amp_rtol = q.loop.rtol;
+    B.phi_rtol = sqrt(q.loop.rtol);
     B.dt = s->dt;
     B.samples = s->samples;
     B.nsamples = s->nsamples;
@@ -294,23 +297,52 @@ int batch_tile(emf_batch *b, int id)
     return EMF_OK;
 }
 
-// The resident solve of member `id` (emf_solve's loop on its own stream).  The
-// handle refuses every other call while it is a member, so its lock is free.
-int batch_resident(emf_batch *b, int id, SolveRun &run)
+// The resident members that have not finished, in order of admission.
+std::vector<int> batch_own(const emf_batch *b)
+{
+    std::vector<int> own;
+    for (int m = 0; m < BATCH_MAX; ++m)
+        if (b->sl[m].s && !b->sl[m].finished && !b->sl[m].tiled) own.push_back(m);
+    std::sort(own.begin(), own.end(), [&](int x, int y) { return b->sl[x].seq < b->sl[y].seq; });
+    return own;
+}
+
+// About `budget` more steps of member `id`'s resident solve (emf_solve's loop on
+// its own stream).  The handle refuses every other call while it is a member, so
+// its lock is free.
+int batch_resident(emf_batch *b, int id, long long &budget)
 {
     BatchSlot &q = b->sl[id];
     HIPCHK(hipSetDevice(b->dev));
-    CHECK(solve_prepare(q.s, q.nmax, q.Tn));
-    CHECK(solve_any(q.s, q.slot, q.rtol, q.nmax, q.Tn, q.fixed_n0, run));
+    CHECK(solve_some(q.s, q.loop, budget));
+    if (q.loop.phase != SolveLoop::DONE) return EMF_OK;
+    const SolveRun &run = q.loop.run;
     q.info.n0 = run.n0;
-    q.info.Tn = q.Tn;
-    q.info.steps = run.n0 + 2 * q.Tn;
+    q.info.Tn = q.loop.Tn;
+    q.info.steps = run.n0 + 2 * q.loop.Tn;
     q.info.status = run.status;
     q.info.nchecks = run.nchecks;
     q.info.a_change = run.a_change;
     q.info.phi_change = run.phi_change;
     q.info.seconds =
         std::chrono::duration<double>(std::chrono::steady_clock::now() - q.t_add).count();
+    q.finished = true;
+    return EMF_OK;
+}
+
+// `replays` replays' worth of steps for the resident members, one after the
+// other in order of admission.  nfin counts those that finish; stops at the first
+// of them if `any`.
+int batch_own_steps(emf_batch *b, long long replays, bool any, int &nfin)
+{
+    b->own_due += replays * b->spg;
+    for (int m : batch_own(b)) {
+        while (b->own_due > 0 && !b->sl[m].finished) CHECK(batch_resident(b, m, b->own_due));
+        if (!b->sl[m].finished) return EMF_OK;
+        ++nfin;
+        if (any) return EMF_OK;
+    }
+    b->own_due = 0;                      // none left
     return EMF_OK;
 }
 
@@ -467,7 +499,9 @@ int emf_batch_add(emf_batch *b, emf_solver *s, int slot, double rtol, double nma
     q.finished = q.tiled = false;
     q.info = emf_solve_info{};
     q.t_add = std::chrono::steady_clock::now();
-    q.rtol = rtol; q.nmax = nmax; q.Tn = Tn; q.fixed_n0 = fixed_n0;
+    q.loop = SolveLoop{};
+    q.loop.slot = slot;
+    q.loop.rtol = rtol; q.loop.nmax = nmax; q.loop.Tn = Tn; q.loop.fixed_n0 = fixed_n0;
     // a member that fits on chip waits for its own resident solve (emf_batch_run)
     const int rc = resident_next(s, ncu, plan) ? solve_prepare(s, nmax, Tn) : batch_tile(b, id);
     if (rc != EMF_OK) {
@@ -495,26 +529,17 @@ int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished)
     BLOCK(b);
     if (max_graphs < 0 || until < 0 || until > 2) EMF_FAIL(EMF_ERR_ARG, "bad arguments");
     int nfin = 0;
-    auto running = [&]() {
+    auto running = [&]() {               // of the members that the graphs step
         int r = 0;
-        for (auto &q : b->sl) r += q.s && !q.finished;
+        for (auto &q : b->sl) r += q.s && q.tiled && !q.finished;
         return r;
     };
     // members that fit on chip: each its own resident solve, a few at once where
     // they leave CUs idle (the gate admits as many boxes as the device has CUs),
-    // and so that one's snapshots and host work overlap another's steps.  A run
-    // of a given number of replays steps them with the others instead.
-    std::vector<int> own;
-    for (int m = 0; m < BATCH_MAX; ++m)
-        if (b->sl[m].s && !b->sl[m].finished && !b->sl[m].tiled) own.push_back(m);
-    std::sort(own.begin(), own.end(), [&](int x, int y) { return b->sl[x].seq < b->sl[y].seq; });
-    if (until == 0 && !own.empty()) {
-        for (int m : own) {
-            std::lock_guard<std::mutex> lks(b->sl[m].s->mtx);
-            CHECK(batch_tile(b, m));
-        }
-        CHECK(batch_sync(b));
-        CHECK(batch_upload_table(b));
+    // and so that one's snapshots and host work overlap another's steps
+    std::vector<int> own = batch_own(b);
+    if (until == 0) {
+        CHECK(batch_own_steps(b, max_graphs, false, nfin));
         own.clear();
     }
     if (until == 1 && own.size() > 1) own.resize(1);
@@ -525,10 +550,13 @@ int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished)
         std::string msg;
         auto work = [&] {
             for (size_t q; (q = next++) < own.size();) {
-                SolveRun run;
-                const int r = batch_resident(b, own[q], run);
+                int r = EMF_OK;
+                while (r == EMF_OK && !b->sl[own[q]].finished) {
+                    long long budget = LLONG_MAX;
+                    r = batch_resident(b, own[q], budget);
+                }
                 std::lock_guard<std::mutex> lk(em);
-                if (r == EMF_OK) { b->sl[own[q]].finished = true; ++nfin; }
+                if (r == EMF_OK) ++nfin;
                 else if (rc == EMF_OK) { rc = r; msg = g_err; }
             }
         };

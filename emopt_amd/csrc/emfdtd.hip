@@ -1323,95 +1323,135 @@ struct SolveRun {
     double a_change = 0, phi_change = 0;
 };
 
-// The solve loop from zero fields: steps until convergence (or fixed_n0 steps),
-// the two snapshots and the phasors.  plan: resident steps, null: the passes.
-int solve_run(emf_solver *s, int slot, double rtol, double nmax, long long Tn, long long fixed_n0,
-              const ResPlan *plan, SolveRun &run)
-{
-    run = SolveRun();
-    // reset CPML and fields (emopt/fdtd.py:1016-1018); set 0 holds step 0
-    set_current(s, 0);
-    CHECK(reset_psi(s));
-    HIPCHK(hipMemsetAsync(s->Ev[0], 0, 3 * s->n * sizeof(double), s->stream));
-    HIPCHK(hipMemsetAsync(s->Hv[0], 0, 3 * s->n * sizeof(double), s->stream));
-    HIPCHK(hipMemsetAsync(s->conv, 0, sizeof(ConvState), s->stream));
-    const double amp_rtol = rtol, phi_rtol = sqrt(rtol);
-    int *dflag = &s->conv->done;
-    // steps [from, from + count); the state after n steps lives in set
-    // from_set(n) (fused) or set 0
-    auto steps = [&](long long from, long long count, const int *done) -> int {
-        if (plan) return res_steps(s, *plan, from, count, done);
-        for (long long q = from; q < from + count; ++q) CHECK(step(s, q, done, from_set(s, q, 0, 0)));
-        return EMF_OK;
-    };
+// A solve loop, which can be left between launches and taken up again: the
+// launches, and so the results, are the same however it is divided.
+struct SolveLoop {
+    int slot = 0;
+    double rtol = 0, nmax = 0;
+    long long Tn = 0, fixed_n0 = -1;
+    bool resident = false;         // resident steps by `plan`, else the step kernels
+    ResPlan plan;
+    enum { START, LOOP, RUN1, RUN2, DONE } phase = START;
+    long long from = 0, pos = 0;   // the run of steps under way: its first step, the next one
+    SolveRun run;
+};
 
-    long long n = 0;
-    if (fixed_n0 >= 0) {
-        CHECK(steps(0, fixed_n0, nullptr));
-        n = fixed_n0;
-        run.status = 2;
-    } else {
-        // The loop breaks at the first step index n > nmax (emopt/fdtd.py:1054).
-        long long n_stop = nmax < 0 ? 0 : (long long)floor(nmax) + 1;
-        const int LOOK = 2;               // chunks in flight before the first flag is read
-        std::vector<std::pair<long long, hipEvent_t>> pend;
-        int ring = 0;
-        while (true) {
-            while ((int)pend.size() < LOOK && Tn > 0 && n + Tn <= n_stop) {
-                // steps after convergence are gated off by dflag and leave the state as is
-                CHECK(steps(n, Tn, dflag));
-                long long nchk = n + Tn - 1;
-                int slotf = ring++ % 32;
-                const int ps = from_set(s, n + Tn, 0, 0);   // set holding E after step nchk
-                hipLaunchKernelGGL(k_conv_check, dim3(1), dim3(64), 0, s->stream, s->Eb[ps][0],
-                                   s->Eb[ps][1], s->Eb[ps][2], s->samples, s->nsamples,
-                                   (double)nchk * s->dt, amp_rtol, phi_rtol, nchk, s->conv,
-                                   s->hist, s->hist_cap, (int *)nullptr);
-                HIPCHK(hipGetLastError());
-                // done and stalled
-                HIPCHK(hipMemcpyAsync(&s->done_host[2 * slotf], dflag, 2 * sizeof(int),
-                                      hipMemcpyDeviceToHost, s->stream));
-                hipEvent_t ev;
-                HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-                HIPCHK(hipEventRecord(ev, s->stream));
-                pend.push_back({ n, ev });
-                n += Tn;
-            }
-            if (pend.empty()) {
-                // fewer than Tn steps remain before nmax: run them and stop
-                CHECK(steps(n, n_stop - n, dflag));
-                n = std::max(n, n_stop);
-                run.status = 1;
-                break;
-            }
-            auto front = pend.front();
-            pend.erase(pend.begin());
-            HIPCHK(hipEventSynchronize(front.second));
-            (void)hipEventDestroy(front.second);
-            int slotf = (ring - 1 - (int)pend.size()) % 32;
-            if (s->done_host[2 * slotf + 1]) { run.stalled = 1; break; }
-            if (s->done_host[2 * slotf]) {
-                n = front.first + Tn;
-                break;
-            }
-        }
-        for (auto &pe : pend) {
-            (void)hipEventSynchronize(pe.second);
-            (void)hipEventDestroy(pe.second);
-        }
-        if (run.stalled) return EMF_OK;
+// Steps L.pos .. end - 1 of the run under way, or as many launches of them as
+// make up `budget` steps, which they are taken from.
+int loop_steps(emf_solver *s, SolveLoop &L, long long end, long long &budget, const int *done)
+{
+    long long k = end - L.pos;
+    if (budget < k) k = std::min(k, (budget + RES_STEPS - 1) / RES_STEPS * RES_STEPS);
+    budget -= k;
+    const long long q0 = L.pos;
+    L.pos += k;
+    if (L.resident) return res_steps(s, L.plan, q0, k, done);
+    // the state after n steps lives in set from_set(n) (fused) or set 0
+    for (long long q = q0; q < q0 + k; ++q) CHECK(step(s, q, done, from_set(s, q, 0, 0)));
+    return EMF_OK;
+}
+
+// The solve loop from where L left it -- zero fields at first: steps until
+// convergence (or fixed_n0 steps), the two snapshots and the phasors -- for
+// about `budget` more steps, whole launches; what is left of them stays in
+// `budget`, negative where the last launch went past.  The work is enqueued; the
+// end of the loop waits for it.
+int solve_advance(emf_solver *s, SolveLoop &L, long long &budget)
+{
+    SolveRun &run = L.run;
+    const long long Tn = L.Tn;
+    if (L.phase == SolveLoop::START) {
+        run = SolveRun();
+        L.from = L.pos = 0;
+        // reset CPML and fields (emopt/fdtd.py:1016-1018); set 0 holds step 0
+        set_current(s, 0);
+        CHECK(reset_psi(s));
+        HIPCHK(hipMemsetAsync(s->Ev[0], 0, 3 * s->n * sizeof(double), s->stream));
+        HIPCHK(hipMemsetAsync(s->Hv[0], 0, 3 * s->n * sizeof(double), s->stream));
+        HIPCHK(hipMemsetAsync(s->conv, 0, sizeof(ConvState), s->stream));
+        L.phase = SolveLoop::LOOP;
     }
-    // capture / two more Tn-step runs / phasor (emopt/fdtd.py:1156-1194)
-    long long n0 = n;
-    set_current(s, from_set(s, n0, 0, 0));
-    CHECK(capture(s, slot, 0));
-    CHECK(steps(n0, Tn, nullptr));
-    set_current(s, from_set(s, n0 + Tn, 0, 0));
-    CHECK(capture(s, slot, 1));
-    CHECK(steps(n0 + Tn, Tn, nullptr));
-    set_current(s, from_set(s, n0 + 2 * Tn, 0, 0));
-    CHECK(phasor3(s, slot, (double)n0 * s->dt, (double)(n0 + Tn) * s->dt,
-                  (double)(n0 + 2 * Tn) * s->dt));
+    if (L.phase == SolveLoop::LOOP) {
+        const bool fixed = L.fixed_n0 >= 0;
+        // The loop breaks at the first step index n > nmax (emopt/fdtd.py:1054).
+        const long long n_stop = fixed ? L.fixed_n0 : (L.nmax < 0 ? 0 : (long long)floor(L.nmax) + 1);
+        int *const dflag = fixed ? nullptr : &s->conv->done;
+        const int LOOK = 2;               // checks in flight before the first flag is read
+        struct Check { long long n; int slot; hipEvent_t ev; };   // after n steps
+        std::vector<Check> pend;
+        int ring = 0, rc = EMF_OK;
+        bool left = false;                // the loop is over
+        auto check = [&]() -> int {
+            const long long nchk = L.pos - 1;
+            const int slotf = ring++ % 32, ps = from_set(s, L.pos, 0, 0);   // set holding E after step nchk
+            hipLaunchKernelGGL(k_conv_check, dim3(1), dim3(64), 0, s->stream, s->Eb[ps][0],
+                               s->Eb[ps][1], s->Eb[ps][2], s->samples, s->nsamples,
+                               (double)nchk * s->dt, L.rtol, sqrt(L.rtol), nchk, s->conv,
+                               s->hist, s->hist_cap, (int *)nullptr);
+            HIPCHK(hipGetLastError());
+            // done and stalled
+            HIPCHK(hipMemcpyAsync(&s->done_host[2 * slotf], dflag, 2 * sizeof(int),
+                                  hipMemcpyDeviceToHost, s->stream));
+            hipEvent_t ev;
+            HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+            pend.push_back({ L.pos, slotf, ev });
+            HIPCHK(hipEventRecord(ev, s->stream));
+            return EMF_OK;
+        };
+        while (rc == EMF_OK && !left && !run.stalled) {
+            // a run of Tn steps with a check after it, or the last one: up to n_stop
+            const bool checked = !fixed && Tn > 0 && L.from + Tn <= n_stop;
+            const long long end = checked ? L.from + Tn : n_stop;
+            const bool may = (int)pend.size() < (checked ? LOOK : 1);
+            if (may && L.pos < end && budget > 0) {
+                // steps after convergence are gated off by dflag and leave the state as is
+                rc = loop_steps(s, L, end, budget, dflag);
+            } else if (may && L.pos >= end && checked) {
+                rc = check();
+                L.from = L.pos;
+            } else if (may && L.pos >= end) {
+                run.n0 = std::max(L.from, n_stop);
+                run.status = fixed ? 2 : 1;
+                left = true;
+            } else if (!pend.empty()) {
+                const Check c = pend.front();
+                pend.erase(pend.begin());
+                if (hipEventSynchronize(c.ev) != hipSuccess) { set_err("check failed"); rc = EMF_ERR_HIP; }
+                (void)hipEventDestroy(c.ev);
+                if (s->done_host[2 * c.slot + 1]) run.stalled = 1;
+                else if (s->done_host[2 * c.slot]) { run.n0 = c.n; left = true; }
+            } else {
+                break;                    // the budget is used up
+            }
+        }
+        for (auto &c : pend) {
+            (void)hipEventSynchronize(c.ev);
+            (void)hipEventDestroy(c.ev);
+        }
+        CHECK(rc);
+        if (!left) return EMF_OK;
+        // capture / two more Tn-step runs / phasor (emopt/fdtd.py:1156-1194)
+        set_current(s, from_set(s, run.n0, 0, 0));
+        CHECK(capture(s, L.slot, 0));
+        L.from = L.pos = run.n0;
+        L.phase = SolveLoop::RUN1;
+    }
+    while (L.phase == SolveLoop::RUN1 || L.phase == SolveLoop::RUN2) {
+        const long long end = L.from + Tn;
+        if (L.pos < end && budget <= 0) return EMF_OK;
+        if (L.pos < end) CHECK(loop_steps(s, L, end, budget, nullptr));
+        if (L.pos < end) continue;
+        set_current(s, from_set(s, end, 0, 0));
+        if (L.phase == SolveLoop::RUN1) {
+            CHECK(capture(s, L.slot, 1));
+            L.from = end;
+            L.phase = SolveLoop::RUN2;
+            continue;
+        }
+        CHECK(phasor3(s, L.slot, (double)run.n0 * s->dt, (double)(run.n0 + Tn) * s->dt,
+                      (double)(run.n0 + 2 * Tn) * s->dt));
+        L.phase = SolveLoop::DONE;
+    }
     // the scalars at the end of the state
     struct { double a_change, phi_change; int done, stalled, nchecks; } cs;
     static_assert(offsetof(ConvState, done) == offsetof(ConvState, a_change) + 16 &&
@@ -1420,14 +1460,12 @@ int solve_run(emf_solver *s, int slot, double rtol, double nmax, long long Tn, l
                                                        offsetof(ConvState, a_change),
                           hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
-    run.n0 = n0;
     run.stalled = cs.stalled;
     run.nchecks = cs.nchecks;
     run.a_change = cs.a_change;
     run.phi_change = cs.phi_change;
     return EMF_OK;
 }
-
 
 // The device state of a solve loop: sample points and check history.
 int solve_prepare(emf_solver *s, double nmax, long long Tn)
@@ -1444,37 +1482,58 @@ int solve_prepare(emf_solver *s, double nmax, long long Tn)
     return EMF_OK;
 }
 
-// solve_run with resident steps where the grid fits, else (or where they
-// stalled) with the step kernels; the history length and the final status.
-int solve_any(emf_solver *s, int slot, double rtol, double nmax, long long Tn, long long fixed_n0,
-              SolveRun &run)
+// solve_advance with resident steps where the grid fits, else (or where they
+// stalled) with the step kernels; at the end the history length and the final
+// status.  Nothing is under way when it returns.
+int solve_some(emf_solver *s, SolveLoop &L, long long &budget)
 {
-    ResPlan plan;
-    int ncu = 0;
-    CHECK(res_cus(s->dev, &ncu));
-    if (resident_next(s, ncu, plan)) {
+    if (L.phase == SolveLoop::START) {
+        int ncu = 0;
+        CHECK(res_cus(s->dev, &ncu));
+        L.resident = resident_next(s, ncu, L.plan);
+    }
+    int rc = EMF_OK;
+    const long long given = budget;
+    if (L.resident) {
         ResHold hold;
-        hold.take(g_res_gate[s->dev], plan.boxes());
-        const int rc = solve_run(s, slot, rtol, nmax, Tn, fixed_n0, &plan, run);
-        if (rc != EMF_OK || run.stalled) (void)hipStreamSynchronize(s->stream);
-        hold.give();
-        CHECK(rc);
-        if (run.stalled) {
+        hold.take(g_res_gate[s->dev], L.plan.boxes());
+        rc = solve_advance(s, L, budget);
+        if (rc != EMF_OK || L.run.stalled || L.phase != SolveLoop::DONE) (void)hipStreamSynchronize(s->stream);
+        hold.give();                           // nothing of it runs any more
+        if (rc == EMF_OK && L.run.stalled) {
             // the work-groups of a launch did not run together: from the start with the passes
             resident_stalled(s);
-            CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
-        } else {
+            L.resident = false;
+            L.phase = SolveLoop::START;
+            budget = given;
+            rc = solve_advance(s, L, budget);
+        } else if (L.phase == SolveLoop::DONE) {
             s->res_row = 0;
         }
     } else {
-        CHECK(solve_run(s, slot, rtol, nmax, Tn, fixed_n0, nullptr, run));
+        rc = solve_advance(s, L, budget);
     }
+    if (rc != EMF_OK) L.phase = SolveLoop::START;      // where it stands is not known
+    CHECK(rc);
+    if (L.phase != SolveLoop::DONE) {
+        HIPCHK(hipStreamSynchronize(s->stream));
+        return EMF_OK;
+    }
+    SolveRun &run = L.run;
     s->nhist = std::min(run.nchecks, s->hist_cap);
     // the loop runs on past non-finite samples (emopt/fdtd.py:1050-1052,
     // 1137-1138) and stops at Nmax: say so when the last check saw them
     if (run.status == 1 && run.nchecks > 0 &&
         !(std::isfinite(run.a_change) && std::isfinite(run.phi_change)))
         run.status = 3;
+    return EMF_OK;
+}
+
+// The whole loop.
+int solve_all(emf_solver *s, SolveLoop &L)
+{
+    for (long long budget = LLONG_MAX; L.phase != SolveLoop::DONE; budget = LLONG_MAX)
+        CHECK(solve_some(s, L, budget));
     return EMF_OK;
 }
 
@@ -2046,8 +2105,11 @@ int emf_solve(emf_solver *s, int slot, double rtol, double nmax, int64_t Tn, int
     CHECK(ensure_slot(s, slot));
     CHECK(solve_prepare(s, nmax, Tn));
     auto t_start = std::chrono::steady_clock::now();
-    SolveRun run;
-    CHECK(solve_any(s, slot, rtol, nmax, Tn, fixed_n0, run));
+    SolveLoop L;
+    L.slot = slot;
+    L.rtol = rtol; L.nmax = nmax; L.Tn = Tn; L.fixed_n0 = fixed_n0;
+    CHECK(solve_all(s, L));
+    const SolveRun &run = L.run;
     auto t_end = std::chrono::steady_clock::now();
     if (info) {
         info->n0 = run.n0;

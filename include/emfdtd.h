@@ -543,7 +543,11 @@ EMF_API int emf_batch_add(emf_batch *b, emf_solver *s, int slot, double rtol, do
 
 /* Replays the graph: until = 0 runs max_graphs replays; 1 returns as soon as
  * a member finishes (or after max_graphs replays); 2 runs until every member
- * has finished.  *finished (may be NULL) = members that finished during the
+ * has finished.  Members whose grid fits on chip (emf_resident when admitted) are
+ * not in the graph: each is its own solve loop of resident launches, the same
+ * as emf_solve's to the bit whatever calls drive it.  For them a replay is
+ * steps_per_graph steps of the first admitted that has not finished, to the next
+ * end of a launch (at most 64 steps).  *finished (may be NULL) = members that finished during the
  * call. */
 EMF_API int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished);
 
