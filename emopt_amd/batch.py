@@ -92,9 +92,11 @@ class Batch:
 
     def run(self, until="all", max_graphs=1 << 30):
         """Replay the step graph.  until = "all" (every member finished),
-        "any" (return at the first finished member) or "graphs" (exactly
-        max_graphs replays).  Finished members are detached; returns their
-        ids."""
+        "any" (return at the first finished member, or after max_graphs
+        replays) or "graphs" (exactly max_graphs replays).  A replay steps
+        resident members as many steps, the first admitted first; "any" takes
+        turns between them and the others.  Finished members are detached;
+        returns their ids."""
         u = {"graphs": 0, "any": 1, "all": 2}[until]
         nf = ctypes.c_int()
         self._lib.emf_batch_run(self._h, int(max_graphs), u, ctypes.byref(nf))

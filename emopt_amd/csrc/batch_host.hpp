@@ -39,6 +39,7 @@ struct BatchSlot {
 
 constexpr int BATCH_LANES_MAX = 4;
 constexpr int BATCH_OWN = 4;             // resident solves at once
+constexpr int BATCH_TURN = 4;            // replays of a turn where resident and other members alternate
 
 struct emf_batch {
     std::mutex mtx;
@@ -54,6 +55,8 @@ struct emf_batch {
     long long group_bytes = 0;          // hot-state bytes per group (0: one group)
     int rotate = 0;                     // 1: groups take turns; 0: first group until done
     long long next_seq = 0;             // admission counter
+    bool own_turn = false;              // resident members are stepped next (batch_until_any)
+    double tile_seconds = 0;            // the graphs' last turn
     long long own_due = 0;              // steps that resident members are due (negative: ahead)
     int ncu = 0;
     BTable *T = nullptr;                // one copy of the table per lane
@@ -340,9 +343,130 @@ int batch_own_steps(emf_batch *b, long long replays, bool any, int &nfin)
         while (b->own_due > 0 && !b->sl[m].finished) CHECK(batch_resident(b, m, b->own_due));
         if (!b->sl[m].finished) return EMF_OK;
         ++nfin;
-        if (any) return EMF_OK;
+        if (any) break;
     }
-    b->own_due = 0;                      // none left
+    b->own_due = std::min(b->own_due, 0LL);   // not kept for members to come
+    return EMF_OK;
+}
+
+// Whether members that the graphs step have not finished.
+bool batch_tiling(const emf_batch *b)
+{
+    for (auto &q : b->sl)
+        if (q.s && q.tiled && !q.finished) return true;
+    return false;
+}
+
+// Replays the graphs: max_graphs times (until 0), or until the first member
+// finishes (1), or until all members that they step have (2, without a limit).
+// nfin counts those that finish.
+int batch_replay(emf_batch *b, long long max_graphs, int until, int &nfin)
+{
+    CHECK(batch_graph(b));
+    // a replay in flight: its lane, snapshot slot, group and end event
+    struct Pend { int lane, r, g; hipEvent_t ev; };
+    std::vector<Pend> pend;
+    int inflight[BATCH_LANES_MAX] = {};
+    long long launched = 0;
+    bool dirty = false, stop = false;
+    int rc = EMF_OK;
+    auto retire = [&](const Pend &p) {
+        if (hipEventSynchronize(p.ev) != hipSuccess) rc = EMF_ERR_HIP;
+        (void)hipEventDestroy(p.ev);
+        --inflight[p.lane];
+        // only the replay's own group: the snapshot was taken while other
+        // lanes were stepping theirs.  The table is the one the replay
+        // ran on (it is only rewritten when nothing is in flight).
+        const BState *snap = b->hS + (size_t)p.r * BATCH_MAX;
+        for (int e = b->hT.gent[p.g]; e < b->hT.gent[p.g + 1]; ++e) {
+            const int m = b->hT.mem[e];
+            BatchSlot &q = b->sl[m];
+            if (q.s && !q.finished && snap[m].phase == BP_DONE) {
+                batch_finish(b, m, snap[m]);
+                ++nfin;
+                dirty = true;
+            }
+        }
+    };
+    while (rc == EMF_OK) {
+        if (until == 1 && nfin > 0) stop = true;
+        if (until == 2 && !batch_tiling(b)) stop = true;
+        if (dirty && !stop) {
+            // compact the work table: wait for the replays in flight first
+            for (auto &p : pend) retire(p);
+            pend.clear();
+            if (rc == EMF_OK) rc = batch_upload_table(b);
+            dirty = false;
+            if (!batch_tiling(b)) stop = true;
+            continue;
+        }
+        // up to two replays in flight per lane, each lane on its group
+        for (int l = 0; l < b->lanes && !stop && rc == EMF_OK; ++l) {
+            while (rc == EMF_OK && inflight[l] < 2 && (until == 2 || launched < max_graphs)) {
+                const int g = batch_lane_group(b, l);
+                if (g < 0) break;
+                hipStream_t st = b->lstream[l];
+                hipEvent_t ev;
+                hipLaunchKernelGGL(k_batch_set_group, dim3(1), dim3(64), 0, st, b->T + l, g);
+                hipError_t le = hipSuccess;
+                if (b->use_graph) le = hipGraphLaunch(b->exec[l], st);
+                else batch_enqueue(b, l);
+                if (hipGetLastError() != hipSuccess || le != hipSuccess ||
+                    hipMemcpyAsync(b->hS + (size_t)b->ring * BATCH_MAX, b->S,
+                                   BATCH_MAX * sizeof(BState), hipMemcpyDeviceToHost,
+                                   st) != hipSuccess ||
+                    hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess ||
+                    hipEventRecord(ev, st) != hipSuccess) {
+                    rc = EMF_ERR_HIP;
+                    break;
+                }
+                pend.push_back({ l, b->ring, g, ev });
+                ++inflight[l];
+                b->ring = (b->ring + 1) % BATCH_RING;
+                ++launched;
+            }
+        }
+        if (pend.empty()) break;
+        const Pend p = pend.front();
+        pend.erase(pend.begin());
+        retire(p);
+    }
+    for (auto &p : pend) retire(p);
+    if (rc == EMF_OK && dirty) rc = batch_upload_table(b);
+    if (rc != EMF_OK) EMF_FAIL(rc, "batch run failed");
+    return EMF_OK;
+}
+
+// Steps until a member finishes, or max_graphs replays of either kind of member
+// are done.  Where there are both, they take turns of BATCH_TURN replays, in order
+// of admission among themselves, and a resident turn lasts as long as the graphs'
+// last one did (their steps take 10 to 50 times as long); whose turn it is
+// outlives the call, so that neither kind waits while the other's members come
+// and go.  In turns, not at once: a resident launch needs all its CUs to itself.
+int batch_until_any(emf_batch *b, long long max_graphs, int &nfin)
+{
+    using clock = std::chrono::steady_clock;
+    long long own_left = max_graphs, tile_left = max_graphs;
+    while (nfin == 0) {
+        const bool own = own_left > 0 && !batch_own(b).empty(), tile = tile_left > 0 && batch_tiling(b);
+        if (!own && !tile) break;
+        const auto t0 = clock::now();
+        auto spent = [&] { return std::chrono::duration<double>(clock::now() - t0).count(); };
+        if (own && (!tile || b->own_turn)) {
+            const long long k = tile ? std::min<long long>(BATCH_TURN, own_left) : own_left;
+            do {
+                CHECK(batch_own_steps(b, k, true, nfin));
+            } while (tile && nfin == 0 && spent() < b->tile_seconds);
+            own_left -= k;
+            b->own_turn = false;
+        } else {
+            const long long k = own ? std::min<long long>(BATCH_TURN, tile_left) : tile_left;
+            CHECK(batch_replay(b, k, 1, nfin));
+            tile_left -= k;
+            b->tile_seconds = spent() * (double)std::min<long long>(BATCH_TURN, k) / (double)k;
+            b->own_turn = true;
+        }
+    }
     return EMF_OK;
 }
 
@@ -529,20 +653,16 @@ int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished)
     BLOCK(b);
     if (max_graphs < 0 || until < 0 || until > 2) EMF_FAIL(EMF_ERR_ARG, "bad arguments");
     int nfin = 0;
-    auto running = [&]() {               // of the members that the graphs step
-        int r = 0;
-        for (auto &q : b->sl) r += q.s && q.tiled && !q.finished;
-        return r;
-    };
+    if (until == 1) {
+        CHECK(batch_until_any(b, max_graphs, nfin));
+        if (finished) *finished = nfin;
+        return EMF_OK;
+    }
     // members that fit on chip: each its own resident solve, a few at once where
     // they leave CUs idle (the gate admits as many boxes as the device has CUs),
     // and so that one's snapshots and host work overlap another's steps
-    std::vector<int> own = batch_own(b);
-    if (until == 0) {
-        CHECK(batch_own_steps(b, max_graphs, false, nfin));
-        own.clear();
-    }
-    if (until == 1 && own.size() > 1) own.resize(1);
+    const std::vector<int> own = until == 2 ? batch_own(b) : std::vector<int>();
+    if (until == 0) CHECK(batch_own_steps(b, max_graphs, false, nfin));
     if (!own.empty()) {
         std::atomic<size_t> next{ 0 };
         std::mutex em;
@@ -570,80 +690,7 @@ int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished)
         for (auto &t : pool) t.join();
         if (rc != EMF_OK) EMF_FAIL(rc, "%s", msg.c_str());
     }
-    if (running() > 0 && !(until == 1 && nfin > 0)) {
-        CHECK(batch_graph(b));
-        // a replay in flight: its lane, snapshot slot, group and end event
-        struct Pend { int lane, r, g; hipEvent_t ev; };
-        std::vector<Pend> pend;
-        int inflight[BATCH_LANES_MAX] = {};
-        int launched = 0;
-        bool dirty = false, stop = false;
-        int rc = EMF_OK;
-        auto retire = [&](const Pend &p) {
-            if (hipEventSynchronize(p.ev) != hipSuccess) rc = EMF_ERR_HIP;
-            (void)hipEventDestroy(p.ev);
-            --inflight[p.lane];
-            // only the replay's own group: the snapshot was taken while other
-            // lanes were stepping theirs.  The table is the one the replay
-            // ran on (it is only rewritten when nothing is in flight).
-            const BState *snap = b->hS + (size_t)p.r * BATCH_MAX;
-            for (int e = b->hT.gent[p.g]; e < b->hT.gent[p.g + 1]; ++e) {
-                const int m = b->hT.mem[e];
-                BatchSlot &q = b->sl[m];
-                if (q.s && !q.finished && snap[m].phase == BP_DONE) {
-                    batch_finish(b, m, snap[m]);
-                    ++nfin;
-                    dirty = true;
-                }
-            }
-        };
-        while (rc == EMF_OK) {
-            if (until == 1 && nfin > 0) stop = true;
-            if (until == 2 && running() == 0) stop = true;
-            if (dirty && !stop) {
-                // compact the work table: wait for the replays in flight first
-                for (auto &p : pend) retire(p);
-                pend.clear();
-                if (rc == EMF_OK) rc = batch_upload_table(b);
-                dirty = false;
-                if (running() == 0) stop = true;
-                continue;
-            }
-            // up to two replays in flight per lane, each lane on its group
-            for (int l = 0; l < b->lanes && !stop && rc == EMF_OK; ++l) {
-                while (rc == EMF_OK && inflight[l] < 2 && (until == 2 || launched < max_graphs)) {
-                    const int g = batch_lane_group(b, l);
-                    if (g < 0) break;
-                    hipStream_t st = b->lstream[l];
-                    hipEvent_t ev;
-                    hipLaunchKernelGGL(k_batch_set_group, dim3(1), dim3(64), 0, st, b->T + l, g);
-                    hipError_t le = hipSuccess;
-                    if (b->use_graph) le = hipGraphLaunch(b->exec[l], st);
-                    else batch_enqueue(b, l);
-                    if (hipGetLastError() != hipSuccess || le != hipSuccess ||
-                        hipMemcpyAsync(b->hS + (size_t)b->ring * BATCH_MAX, b->S,
-                                       BATCH_MAX * sizeof(BState), hipMemcpyDeviceToHost,
-                                       st) != hipSuccess ||
-                        hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess ||
-                        hipEventRecord(ev, st) != hipSuccess) {
-                        rc = EMF_ERR_HIP;
-                        break;
-                    }
-                    pend.push_back({ l, b->ring, g, ev });
-                    ++inflight[l];
-                    b->ring = (b->ring + 1) % BATCH_RING;
-                    ++launched;
-                }
-            }
-            if (pend.empty()) break;
-            const Pend p = pend.front();
-            pend.erase(pend.begin());
-            retire(p);
-        }
-        for (auto &p : pend) retire(p);
-        if (rc == EMF_OK && dirty) rc = batch_upload_table(b);
-        if (rc != EMF_OK) EMF_FAIL(rc, "batch run failed");
-    }
+    if (batch_tiling(b)) CHECK(batch_replay(b, max_graphs, until, nfin));
     if (finished) *finished = nfin;
     return EMF_OK;
 }

@@ -12,9 +12,10 @@ Admission is first-come first-served: the queue head waits until it fits
 (no overtaking, so no request starves).  At most `max_running` solves are
 members of the batch; up to `prep_ahead` more are built ahead on the
 workers, so a finished solve is replaced at the next replay boundary.  The
-batch steps its members in cache-sized groups in admission order, the
-oldest group first, so the device works through requests in arrival order
-while the host builds the next ones.  Results do not depend on admission
+batch steps requests that fit on chip one after the other in admission order,
+and larger ones in cache-sized groups, the oldest group first; the two kinds take
+turns of a few replays, so neither starves while the other's requests keep
+coming.  The host builds the next requests meanwhile.  Results do not depend on admission
 order or on the other requests in the batch: each member's arithmetic is its
 own.
 """

@@ -547,7 +547,10 @@ EMF_API int emf_batch_add(emf_batch *b, emf_solver *s, int slot, double rtol, do
  * not in the graph: each is its own solve loop of resident launches, the same
  * as emf_solve's to the bit whatever calls drive it.  For them a replay is
  * steps_per_graph steps of the first admitted that has not finished, to the next
- * end of a launch (at most 64 steps).  *finished (may be NULL) = members that finished during the
+ * end of a launch (at most 64 steps).  Where there are members of both kinds,
+ * until = 1 steps them in turns of at most 4 replays, also from call to call, and
+ * a resident turn lasts as long as the graph's last one (max_graphs bounds either
+ * kind's replays, and so the call); until = 2 takes the resident ones first.  *finished (may be NULL) = members that finished during the
  * call. */
 EMF_API int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished);
 

@@ -99,3 +99,57 @@ def test_stall_between_calls():
         got = _driven(cases, dict(fixed_n0=300), graphs, resident=(1, 1))[0]
         assert got[0] == ref[0]
         assert max(rel_l2(x, y) for x, y in zip(got[2], ref[2])) <= TOL
+
+
+def test_any_is_bounded_by_replays():
+    """until="any" returns after max_graphs replays where no member has finished."""
+    from emopt_amd.batch import Batch
+    cases = [batch_case(q, n_fwd=2, **SMALL) for q in (0, 1)]
+    whole = _driven(cases, dict(fixed_n0=200), [])
+    b = Batch(steps_per_graph=16)
+    sims = [_sim(c, dict(fixed_n0=200)) for c in cases]
+    for s in sims:
+        b.add(s, postprocess=False)
+    calls, done = 0, []
+    while b.running:
+        done += [(m, calls) for m in b.run(until="any", max_graphs=2)]
+        calls += 1
+        assert calls < 100
+    assert [m for m, _ in done] == [0, 1]
+    steps = [200 + 2 * s.Tn for s in sims]
+    assert abs(32 * done[0][1] - steps[0]) <= 96       # a call, and a launch
+    assert abs(32 * done[1][1] - sum(steps)) <= 160    # and the call that ended with the first
+    b.close()
+    for s, c, ref in zip(sims, cases, whole):
+        _same(_result(s, c), ref)
+
+
+def test_neither_kind_of_member_waits_for_ever():
+    """A member that the graphs step finishes while members that fit on chip keep
+    coming, and they while it runs; the results are those of each alone."""
+    from emopt_amd.batch import Batch
+    big, small = batch_case(0, n_fwd=2, **SMALL), batch_case(1, n_fwd=2, **SMALL)
+    ref_big = _driven([big], dict(fixed_n0=600), [], spg=16, resident=(0, 0))[0]
+    ref_small = _driven([small], dict(fixed_n0=20), [], spg=16)[0]
+    b = Batch(steps_per_graph=16)
+    sim = _sim(big, dict(fixed_n0=600), (0, 0))
+    mid = b.add(sim, postprocess=False)
+    limit = 3 * (600 + 2 * sim.Tn) // (4 * 16) + 4     # a turn of 4 replays in 3 calls
+    live, got = {}, []
+    for calls in range(limit):
+        if not live:
+            s = _sim(small, dict(fixed_n0=20))
+            live[b.add(s, postprocess=False)] = s
+        done = b.run(until="any", max_graphs=4)
+        got += [live.pop(m) for m in done if m in live]
+        if mid in done:
+            break
+    else:
+        pytest.fail("the graphs' member has not finished after %d calls" % limit)
+    print("big member done after %d of %d calls, %d small ones" % (calls + 1, limit, len(got)))
+    assert len(got) >= 2
+    b.run()
+    b.close()
+    _same(_result(sim, big), ref_big)
+    for s in got:
+        _same(_result(s, small), ref_small)
