@@ -6,8 +6,8 @@ every member's solve loop (emopt/fdtd.py:994-1194) runs on the device, so the
 host only replays a captured hipGraph of ``steps_per_graph`` steps and reads
 the members' states between replays.  A member whose grid fits on chip takes
 its own resident solve instead, as ``solve_forward`` does: 5 to 10 us per step of
-up to 655,000 cells.  Members may
-be added while others run (continuous batching).  A member's fields agree with those of
+up to 655,000 cells, 15 to 30 up to 1.3 million.  Members may be added while others
+run (continuous batching).  A member's fields agree with those of
 ``solve_forward`` / ``solve_adjoint`` on the same problem to roundoff (same
 n0 and step counts; to the bit where it is resident), and do not depend on the
 other members, nor on how ``run`` was called.

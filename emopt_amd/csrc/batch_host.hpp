@@ -38,7 +38,7 @@ struct BatchSlot {
 }  // namespace
 
 constexpr int BATCH_LANES_MAX = 4;
-constexpr int BATCH_OWN = 4;             // resident solves at once
+constexpr int BATCH_OWN = 4;             // threads for resident solves
 constexpr int BATCH_TURN = 4;            // replays of a turn where resident and other members alternate
 
 struct emf_batch {
@@ -658,9 +658,9 @@ int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished)
         if (finished) *finished = nfin;
         return EMF_OK;
     }
-    // members that fit on chip: each its own resident solve, a few at once where
-    // they leave CUs idle (the gate admits as many boxes as the device has CUs),
-    // and so that one's snapshots and host work overlap another's steps
+    // members that fit on chip: each its own resident solve.  The gate admits them
+    // one after the other where each takes more than half of the CUs, as nearly all
+    // grids do; the threads start one as soon as another ends
     const std::vector<int> own = until == 2 ? batch_own(b) : std::vector<int>();
     if (until == 0) CHECK(batch_own_steps(b, max_graphs, false, nfin));
     if (!own.empty()) {

@@ -22,11 +22,12 @@
 // the faces the producer needs to reach step s + 2 and reuse the slot.
 //
 // All work-groups have to run at the same time: the grid has at most one per
-// CU, and the host admits no more work-groups of such launches than CUs at
-// once.  Where they still do not (another process holding CUs with a launch of
-// the same kind), a poll gives up after RES_SPIN tries, sets conv->stalled and
-// every work-group runs through without waiting; the host then repeats the
-// solve with the two passes.
+// CU, and the host admits launches together only where each XCD has a CU for all of
+// their work-groups on it (ResGate).  Where they still do not run (another process
+// holding CUs with a launch of the same kind), a poll gives up after RES_SPIN
+// tries, sets conv->stalled and every work-group runs through without waiting; the
+// host then repeats the solve with the two passes, and tries resident steps again
+// some solves later.
 #pragma once
 #include "twopass.hpp"
 
@@ -151,7 +152,10 @@ __global__ __launch_bounds__(RES_T, 2) void k_resident(ResArgs R, FusedArgs A, G
     const int x0 = bx * Nx / GX, xw = (bx + 1) * Nx / GX - x0;
     const int y0 = by * Ny / GY, yw = (by + 1) * Ny / GY - y0;
     const int z0 = bz * Nz / GZ, zw = (bz + 1) * Nz / GZ - z0;
-    const bool full = zw == NZ;       // planes: NZ, or NZ - 1 with a spare one that holds zeros
+    // planes: NZ, or NZ - 1 with a spare one on top.  Its E stays zero (no coefficients);
+    // its H does not, but only the spare plane's own E and the neighbours' spare
+    // planes read it.
+    const bool full = zw == NZ;
     const int p = (int)threadIdx.x, nt = (int)blockDim.x;
     const bool on = p < xw * yw;
     const int y = on ? p / xw : 0, x = on ? p - y * xw : 0;

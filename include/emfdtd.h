@@ -376,8 +376,9 @@ EMF_API int emf_set_tuning(emf_solver *s, int kind, int tyg, int zc, int order);
 EMF_API int emf_set_wide_offsets(emf_solver *s, int force);
 
 /* Resident steps: a solve (emf_solve) with step kernel kind 1 whose grid fits
- * the chip's registers (up to about 655,000 cells with real eps and uniform
- * mu, 393,000 otherwise) takes many steps per launch with its state on chip.
+ * the chip's registers (up to about 1.3 million cells, with psi and coefficients
+ * in memory from 655,000 on, with complex eps from 393,000; 393,000 with a mu array)
+ * takes many steps per launch with its fields on chip.
  * on = 0 keeps such a solve on the step kernels; spin > 0 bounds the polls for
  * a neighbour's data before the launch counts as stalled (something else held
  * CUs of the device meanwhile) and the solve is repeated with the step kernels
