@@ -1767,6 +1767,7 @@ int emf_set_mat_arrays(emf_solver *s, const double *ex, const double *ey, const 
                                   s->stream));
         }
     HIPCHK(hipStreamSynchronize(s->stream));
+    s->cidx_valid = false;         // also where no new index is built now
     if (s->compress) CHECK(build_coeff_index(s));
     s->mat_set = true;
     s->coef_dirty = true;
