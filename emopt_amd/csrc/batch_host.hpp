@@ -683,8 +683,8 @@ int emf_batch_run(emf_batch *b, int max_graphs, int until, int *finished)
         std::vector<std::thread> pool;
         try {
             for (size_t t = 1; t < std::min<size_t>(own.size(), BATCH_OWN); ++t) pool.emplace_back(work);
-        } catch (const std::system_error &) {
-            // no more threads: those there are (this one at least) take all members
+        } catch (const std::exception &) {
+            // no more threads, or no memory for one: those there are (this one at least) take all members
         }
         work();
         for (auto &t : pool) t.join();

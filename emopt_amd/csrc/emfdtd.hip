@@ -20,9 +20,9 @@
 #include <cstdio>
 #include <cstring>
 #include <condition_variable>
+#include <exception>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 

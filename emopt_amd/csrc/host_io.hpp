@@ -137,8 +137,8 @@ void in_threads(int n, F &&f)
     int started = 1;
     try {
         for (; started < n; ++started) pool.emplace_back([&f, t = started] { f(t); });
-    } catch (const std::system_error &) {
-        // no more threads: the rest run here
+    } catch (const std::exception &) {
+        // no more threads, or no memory for one: the rest run here
     }
     f(0);
     for (int t = started; t < n; ++t) f(t);

@@ -19,7 +19,7 @@ STAND_IN = r"""
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 typedef int hipError_t;
@@ -109,6 +109,34 @@ int main()
         pool_leave(0);
     }
     EXPECT(slabs == 0 && streams == 0 && events == 0);
+    return 0;
+}
+""")
+
+
+def test_work_is_done_where_threads_are_not_to_be_had(tmp_path):
+    """Out of memory at each allocation that starting the threads makes."""
+    _run(tmp_path, """
+#include <new>
+static std::atomic<int> left{ -1 };
+void *operator new(size_t n)
+{
+    if (left >= 0 && left-- == 0) throw std::bad_alloc();
+    void *p = malloc(n);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+int main()
+{
+    for (int at = 0; at < 12; ++at) {
+        std::atomic<int> runs[4]{};
+        left = at;
+        in_threads(4, [&](int t) { ++runs[t]; });
+        left = -1;
+        for (auto &r : runs) EXPECT(r == 1);
+    }
     return 0;
 }
 """)
